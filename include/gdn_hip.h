@@ -366,8 +366,9 @@ int gdn_prefill_split_h_fwd(const uint16_t* q, const uint16_t* k, const uint16_t
  * produces, kernel.py:1153-1160, here gdn_prefill_h_fwd).
  *
  * Device workspace bytes of gdn_prefill_bwd: per (64-token chunk slot,
- * v-head) 96 KiB (the chunk's state-gradient transition and the gradient of
- * the state leaving it).  0 for invalid sizes.
+ * v-head) 72 KiB (the chunk's state-gradient transition, whose second half
+ * becomes the gradient of the state leaving it, and the chunk's triangular
+ * inverse) and 8 bytes per slot.  0 for invalid sizes.
  */
 size_t gdn_prefill_bwd_workspace_bytes(int N, int T, int HQ, int HV);
 
@@ -389,7 +390,7 @@ size_t gdn_prefill_bwd_workspace_bytes(int N, int T, int HQ, int HV);
  *                gdn_gate_bwd maps them to a, b, A_log, dt_bias.
  *   d_initial_state : [N, HV, 128, 128], or NULL when not wanted.
  * Products take bf16 operands with fp32 accumulation.  Three launches
- * (plus one when HV > HQ) on `stream`: per-chunk state-gradient transitions
+ * on `stream`: per-chunk state-gradient transitions
  * (all chunks at once), the chain over each sequence's chunks in reverse,
  * and the per-chunk gradients.  Not q/k L2-normalising (GDN_QK_L2NORM has no
  * backward here).  GDN_ERR_WORKSPACE when the workspace is NULL or short.

@@ -1,0 +1,48 @@
+"""The training step's backward (one call through the gating, bf16 token
+gradients) against gdn_prefill_backward and gdn_gate_backward.
+
+The two share every kernel up to the final store, so a token gradient equals
+the fp32 one rounded to bf16 bit for bit.  dA_log and ddt_bias sum the same
+fp32 terms in another order: T terms of either sign, each sum within T 2^-24
+of the terms' magnitudes, so the two agree within 2 T 2^-24 sum |term|.
+"""
+
+import pytest
+import torch
+
+from conftest import pkg_module
+
+pytestmark = pytest.mark.gpu
+
+
+# single tokens and lengths around a chunk (rows past the end of every tile),
+# empty sequences, G = 1, 2, 4, no sequence at all, more units than CUs
+@pytest.mark.parametrize("lens,HQ,HV,with_state,dfin,cu32", [
+    ([1], 4, 8, True, True, False), ([15, 16, 17], 1, 4, True, False, True),
+    ([63, 64, 65], 4, 4, False, True, False), ([0, 130, 0], 2, 4, True, True, True),
+    ([700, 33], 16, 32, False, False, False), ([], 4, 8, False, False, False)])
+def test_step_equals_separate_calls(device, lens, HQ, HV, with_state, dfin, cu32):
+    print(f"backward step lens={lens} HQ={HQ} HV={HV}", flush=True)
+    inp, pre, bwd = (pkg_module(n) for n in ("inputs", "prefill", "backward"))
+    x = inp.prefill_inputs(lens, HQ, HV, seed=5 + sum(lens), with_state=with_state,
+                           cu_dtype=torch.int32 if cu32 else torch.int64)
+    g = {k: (v.to(device) if torch.is_tensor(v) else v) for k, v in x.items()}
+    T, N = sum(lens), len(lens)
+    gen = torch.Generator(device=device).manual_seed(17)
+    d_out = torch.randn(T, HV, 128, generator=gen, device=device).to(torch.bfloat16)
+    d_fin = torch.randn(N, HV, 128, 128, generator=gen, device=device) * 0.1 if dfin else None
+    head = (g["q"], g["k"], g["v"])
+    gates = (g["A_log"], g["a"], g["dt_bias"], g["b"])
+    _, _, h = pre.gdn_prefill_h(*head, g["state"], *gates, g["cu_seqlens"], g["scale"])
+    want = bwd.gdn_prefill_backward(*head, *gates, g["cu_seqlens"], g["scale"], h, d_out, d_fin)
+    gate = bwd.gdn_gate_backward(*gates, want["dg"], want["dbeta"])
+    dq, dk, dv, dA_log, da, ddt_bias, db, dh0 = bwd._step_backward(
+        *head, *gates, g["cu_seqlens"], g["scale"], h, d_out, d_fin, True)
+    torch.cuda.synchronize()
+    for got, ref in ((dq, want["dq"]), (dk, want["dk"]), (dv, want["dv"]), (da, gate["da"]), (db, gate["db"])):
+        assert torch.equal(got, ref.to(torch.bfloat16))
+    assert torch.equal(dh0, want["dh0"])
+    # |dg g| and |da| per head: the gate backward of |dg|
+    size = bwd.gdn_gate_backward(*gates, want["dg"].abs(), want["dbeta"])
+    for got, name in ((dA_log, "dA_log"), (ddt_bias, "ddt_bias")):
+        assert bool(((got - gate[name]).abs() <= 2 * T * 2.0 ** -24 * size[name].abs()).all()), name

@@ -25,7 +25,8 @@ GDN_PREFILL_PLAN_BYTES = 512
 GDN_ACT_NONE = 0
 GDN_ACT_SILU = 1
 
-# Every symbol include/gdn_hip.h declares, with (restype, argtypes).
+# Every symbol include/gdn_hip.h and csrc/gdn_backward_step.h declare, with
+# (restype, argtypes).
 _P = ctypes.c_void_p
 _I = ctypes.c_int
 _F = ctypes.c_float
@@ -67,6 +68,8 @@ SIGNATURES = {
     "gdn_prefill_bwd_workspace_bytes": (_S, [_I, _I, _I, _I]),
     "gdn_prefill_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _P,
                              _P, _P, _P, _P, _P, _P, _P, _P, _S, _P]),
+    "gdn_prefill_bwd_step": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I,
+                                  _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _S, _P]),
     "gdn_gate_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P, _P, _P]),
 }
 

@@ -35,8 +35,9 @@ HEAD_SIZE = 128
 
 def workspace_bytes(N: int, T: int, HQ: int, HV: int) -> int:
     """Device workspace of :func:`gdn_prefill_backward`: per chunk slot and
-    v-head the chunk's state-gradient transition (M and R, 32 KiB bf16 each)
-    and the gradient of the state leaving it (32 KiB bf16)."""
+    v-head the chunk's state-gradient transition (M and R, 32 KiB bf16 each;
+    the gradient of the state leaving the chunk then takes R's place) and its
+    triangular inverse (8 KiB bf16), and 8 bytes per chunk slot."""
     return int(_capi.lib().gdn_prefill_bwd_workspace_bytes(N, T, HQ, HV))
 
 
@@ -122,16 +123,45 @@ def gdn_gate_backward(A_log, a, dt_bias, b, dg, dbeta):
     return out
 
 
+def _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, scale, h, d_out, d_final_state,
+                   need_initial_state_grad: bool):
+    """The gradients of one training step in the inputs' own types: the token
+    gradients in bf16 (rounded once, where they are formed), ``dA_log``,
+    ``ddt_bias`` and the initial state's in fp32."""
+    T, HQ, _ = q.shape
+    HV = v.shape[1]
+    N = cu_seqlens.numel() - 1
+    dev = q.device
+    q, k, v, a, b, A_log, dt_bias, cu, h = (t.contiguous() for t in (q, k, v, a, b, A_log, dt_bias,
+                                                                     cu_seqlens, h))
+    d_out = d_out.to(torch.bfloat16).contiguous()
+    if d_final_state is not None:
+        d_final_state = d_final_state.to(torch.float32).contiguous()
+    grads = [torch.empty(t.shape, dtype=torch.bfloat16, device=dev) for t in (q, k, v, a, b)]
+    dA_log, ddt_bias = (torch.empty(HV, dtype=torch.float32, device=dev) for _ in range(2))
+    dh0 = (torch.empty(N, HV, HEAD_SIZE, HEAD_SIZE, dtype=torch.float32, device=dev)
+           if need_initial_state_grad else None)
+    ws = torch.empty(max(workspace_bytes(N, T, HQ, HV), 1), dtype=torch.uint8, device=dev)
+    p = _capi.ptr
+    rc = _capi.lib().gdn_prefill_bwd_step(
+        p(q), p(k), p(v), p(A_log), p(a), p(dt_bias), p(b), p(cu),
+        1 if cu.dtype == torch.int32 else 0, N, T, HQ, HV, float(scale), p(h), h.shape[0],
+        p(d_out), p(d_final_state), *[p(t) for t in grads], p(dA_log), p(ddt_bias), p(dh0), p(ws),
+        ws.numel(), _capi.stream_handle(dev))
+    _capi.check(rc, "gdn_prefill_bwd_step")
+    dq, dk, dv, da, db = grads
+    return dq, dk, dv, dA_log, da, ddt_bias, db, dh0
+
+
 class _GatedDeltaRule(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, A_log, a, dt_bias, b, initial_state, cu_seqlens, scale):
         o, final, h = _pre.gdn_prefill_h(q, k, v, initial_state, A_log, a, dt_bias, b,
                                          cu_seqlens, scale)
         ctx.save_for_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, h)
-        ctx.scale = scale
+        ctx.scale = _pre._resolve_scale(scale)
         ctx.has_state = initial_state is not None
-        ctx.dtypes = (q.dtype, k.dtype, v.dtype, A_log.dtype, a.dtype, dt_bias.dtype, b.dtype,
-                      None if initial_state is None else initial_state.dtype)
+        ctx.set_materialize_grads(False)       # no zeros for an output without a gradient
         return o, final
 
     @staticmethod
@@ -139,13 +169,11 @@ class _GatedDeltaRule(torch.autograd.Function):
         q, k, v, A_log, a, dt_bias, b, cu_seqlens, h = ctx.saved_tensors
         if d_o is None:
             d_o = torch.zeros(v.shape, dtype=torch.bfloat16, device=v.device)
-        g = gdn_prefill_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, ctx.scale, h, d_o,
-                                 d_final, need_initial_state_grad=ctx.has_state)
-        gg = gdn_gate_backward(A_log, a, dt_bias, b, g["dg"], g["dbeta"])
-        tq, tk, tv, tA, ta, tdt, tb, ts = ctx.dtypes
-        ds = g["dh0"].to(ts) if ctx.has_state else None
-        return (g["dq"].to(tq), g["dk"].to(tk), g["dv"].to(tv), gg["dA_log"].to(tA),
-                gg["da"].to(ta), gg["ddt_bias"].to(tdt), gg["db"].to(tb), ds, None, None)
+        # the forward takes bf16 q, k, v, a, b and fp32 A_log, dt_bias, state only
+        with torch.no_grad():
+            grads = _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, ctx.scale, h, d_o,
+                                   d_final, ctx.has_state)
+        return grads + (None, None)
 
 
 def chunk_gated_delta_rule(q, k, v, A_log, a, dt_bias, b, cu_seqlens, initial_state=None,

@@ -19,25 +19,29 @@
 //        M = e^{gam_L} I - W2^T (beta E K),   W2 = Tm^T Dc K            [K x K]
 //        R = dO^T (scale E Q) - G1^T (beta E K),  G1 = Tm^T P^T dO      [V x K]
 //     so that dS = dSn M + R.  M is written as ready MFMA A-operand
-//     fragments, R in the accumulator layout of the chain kernel.
+//     fragments, R in the accumulator layout of the chain kernel, and Tm for
+//     the gradient kernel.
 //  2. gdn_bwd_chain_kernel, one workgroup per (sequence, v-head), or per
 //     quarter of its state rows when the chains are few: walks the chunks
 //     from last to first with dS^T in MFMA accumulators, storing dSn of
 //     every chunk (bf16) and the gradient of the initial state.
-//  3. gdn_bwd_grad_kernel, one workgroup per (chunk, qk-head), its v-heads
-//     in turn: with S and dSn known, every gradient of the chunk:
+//  3. gdn_bwd_grad_kernel, persistent workgroups over the (chunk, qk-head)
+//     units, a unit's v-heads in turn: with S and dSn known, every gradient
+//     of the chunk:
 //        dVn = P^T dO + Dc K dSn^T,  dX = Tm^T dVn,  dV = beta dX,
-//        dP = dO Vn^T,  dTm = dVn X^T,  dA = -Tm^T dTm Tm^T (strictly lower),
+//        dP = dO Vn^T,  dA = -dX Vn^T (strictly lower),
 //        dQ = scale E dO S + dPm K,
-//        dK = Dc Vn dSn - beta E dX S + dPm^T Q + dAb K + dAb^T K,
+//        dK = Dc Vn dSn - beta E dX S + dPm^T Q + (dAb + dAb^T) K,
 //        dbeta = rowsum(dA Ar) + rowsum(dX (V - E K S^T)),
 //        dgam  = rowsum - colsum of (dP P) and of (dA A) + scale E rowsum(Q (dO S))
 //                - beta E rowsum(dX K S^T) - Dc rowsum(Vn K dSn^T)
 //                (+ sum_i Dc rowsum(Vn K dSn^T) + e^{gam_L} <dSn, S> at gam_L),
 //        dg = reverse cumsum of dgam within the chunk,
 //     with dPm = scale e^{gam_i-gam_j} dP (j <= i), dAb = beta_i e^{gam_i-gam_j} dA.
-//     dq / dk of the v-heads that share a qk-head are summed in registers,
-//     in v-head order, and stored once.
+//     (dA is the inverse's gradient -Tm^T (dVn X^T) Tm^T: its outer factors
+//     turn dVn into dX and X into Vn, so neither dVn X^T nor the two 64^3
+//     products around it are formed.)  dq / dk of the v-heads that share a
+//     qk-head are summed in registers, in v-head order, and stored once.
 //
 // All products run on MFMA 16x16x32 bf16 with fp32 accumulation; the matrix
 // operands live in LDS as bf16 rows of the form [m][r] and are read either
@@ -51,6 +55,7 @@
 
 #include "gdn_prefill_common.h"
 #include "gdn_prefill_split.h"
+#include "gdn_backward_step.h"
 #include "../../include/gdn_hip.h"
 
 #include <algorithm>
@@ -65,8 +70,8 @@ constexpr int LDA = C + 4;           // [64][64] fp32 rows (272 B)
 constexpr int kCB = C * LDK;         // elements of a [64][128] buffer
 constexpr int kTB = C * LDC;         // elements of a [64][64] buffer
 constexpr size_t kMBytes = size_t(D) * D * 2;   // M record (bf16 fragments)
-constexpr size_t kRBytes = size_t(D) * D * 2;   // R record (bf16, accumulator layout)
-constexpr size_t kHBytes = size_t(D) * D * 2;   // dSn record (bf16 [v][k])
+constexpr size_t kRBytes = size_t(D) * D * 2;   // R record (bf16, accumulator layout); then dSn (bf16 [v][k])
+constexpr size_t kTmBytes = size_t(C) * C * 2;  // Tm record (bf16 [t][t'], zero above the diagonal)
 constexpr int kGradThreads = 512;
 
 typedef short i16x8_t __attribute__((ext_vector_type(8)));
@@ -99,17 +104,21 @@ __device__ __forceinline__ void st_tile(uint16_t* base, int ld, int r0, int c0, 
   for (int i = 0; i < 4; ++i) p[i * ld] = f32_to_bf16_bits(x[i]);
 }
 
-// Sum over the 4 lane groups (same lane % 16) of a wave.
+// Sum over the 4 lane groups (same lane % 16) of a wave, in every lane: a
+// permlane swap of a value with itself leaves one half's values in all lanes
+// of one result and the other half's in the other.
 __device__ __forceinline__ float group4_sum(float x) {
-  x += __shfl_xor(x, 16);
-  x += __shfl_xor(x, 32);
-  return x;
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // Gate data of one chunk in LDS: gam | beta | e^gam | e^{gam_L - gam} (64 each),
 // then gam_L, e^{gam_L}.  Wave-0 work: lane t takes token t of the chunk.
 constexpr int GB_GAM = 0, GB_BETA = C, GB_E = 2 * C, GB_DC = 3 * C, GB_L = 4 * C, GB_EL = 4 * C + 1;
 constexpr int GB_SZ = 4 * C + 4;
+constexpr int GB_DA = GB_SZ, GB_DB = GB_SZ + C, GB_G = GB_SZ + 2 * C;   // GateFactors (training step only)
 
 // The gate inputs of token `lane` of the chunk (wave 0): loaded early, used
 // by chunk_gates_calc once the chunk's rows are on their way.
@@ -310,7 +319,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_prep_kernel(
     const uint16_t* __restrict__ a, const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
     const CuT* __restrict__ cu, int N, int T, int HQ, int HV, float scale,
     const uint16_t* __restrict__ d_out, int h_chunks, int slots, char* __restrict__ mrec,
-    char* __restrict__ rrec) {
+    char* __restrict__ rrec, uint16_t* __restrict__ tmrec, int2* __restrict__ chunks) {
   __shared__ __align__(16) uint16_t sK[kCB];      // K; then G0 = P^T dO
   __shared__ __align__(16) uint16_t sQ[kCB];      // Q; then W2 = Tm^T Dc K
   __shared__ __align__(16) uint16_t sdO[kCB];
@@ -358,6 +367,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_prep_kernel(
   bool ok = int(blockIdx.x) < units && locate(int(blockIdx.x), t0, len);
   if (ok) fetch(int(blockIdx.x), t0, len, wk, wq, wo, gi);
   for (int u = int(blockIdx.x); u < units; u += int(gridDim.x)) {
+    // the slot's token range for the gradient kernel (length 0: no chunk)
+    if (u < slots && tid0 == 0) chunks[u] = int2{t0, ok ? len : 0};
     // the next unit's inputs, in flight while this one is worked on
     const int un = u + int(gridDim.x);
     int t0n = 0, lenn = 0;
@@ -419,6 +430,9 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_prep_kernel(
       }
       lds_barrier();
 
+      // Tm for the gradient kernel
+      reinterpret_cast<uint4*>(tmrec + (size_t(slot) * HV + hv) * C * C)[tid] =
+          *reinterpret_cast<const uint4*>(sTm + (tid >> 3) * LDC + 8 * (tid & 7));
       // W2 = Tm^T Dc K -> sQ, -G1 = -Tm^T G0 -> sAr (as bf16 [64][LDK])
       uint16_t* sG1 = reinterpret_cast<uint16_t*>(sAr);
       {
@@ -495,15 +509,16 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_prep_kernel(
 
 // ---------------------------------------------------------------------------
 // 2. The state-gradient chain per (sequence, v-head), last chunk first:
-//    dh[chunk] = dSn (bf16 [v][k]);  dS = dSn M + R;  finally dh0 = dS.
+//    dS = dSn M + R, dSn (bf16 [v][k]) over the chunk's R record;  finally dh0 = dS.
+// The 16 rows of dSn that a wave writes are the bytes of the R block that only
+// it reads, and it has them in registers by then.
 // NW waves per workgroup, 128 / (16 NW) workgroups per chain.  A wave keeps
 // dS^T[k][v] for its 16 state rows v as 8 accumulator tiles (k blocks); the
 // B operand of step s is the pair of tiles kt = 2 s, 2 s + 1.
 template <typename CuT, int NW>
 __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     const CuT* __restrict__ cu, int N, int T, int HV, int h_chunks, const char* __restrict__ mrec,
-    const char* __restrict__ rrec, const float* __restrict__ d_ht, uint16_t* __restrict__ dh,
-    float* __restrict__ dh0) {
+    char* rrec, const float* __restrict__ d_ht, float* __restrict__ dh0) {
   constexpr int S = 8 / NW;                    // slices (of 16 NW state rows) per chain
   constexpr int kThreads = 64 * NW;
   __shared__ __align__(16) uint16_t sM[3][D * D];
@@ -560,7 +575,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
       copy_m(ch - 2, (it + 2) % 3);
       fetch_r(ch - 2, nxt2);
     }
-    uint16_t* hd = dh + rec_of(ch) * D * D;
+    uint16_t* hd = reinterpret_cast<uint16_t*>(rrec + rec_of(ch) * kRBytes);
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
       uint2 w;
@@ -609,400 +624,640 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
   }
 }
 
+// Gradients of one token's gating
+//   g = -exp(A_log) softplus(x), x = a + dt_bias;  beta = sigmoid(b):
+//   da = dg (-exp(A_log) sigmoid(x)) (ddt_bias sums them),  db = dbeta beta (1 - beta),
+//   dA_log sums dg g.  The factors of dg and dbeta:
+struct GateFactors {
+  float da, db, g;
+};
+__device__ __forceinline__ GateFactors gate_factors(float x, float b, float exp_a) {
+  const float be = sigmoidf_(b);
+  return GateFactors{-exp_a * sigmoidf_(x), be * (1.f - be), -exp_a * softplus_stable(x)};
+}
+
+// Sums of x and of y over a workgroup of 256 threads, whole in thread 0.
+__device__ __forceinline__ void sum_pair_256(float& x, float& y, float (&red)[2][4]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    x += __shfl_xor(x, off);
+    y += __shfl_xor(y, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = x;
+    red[1][threadIdx.x >> 6] = y;
+  }
+  __syncthreads();
+  x = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+  y = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+}
+
 // ---------------------------------------------------------------------------
 // 3. Gradients of one (chunk, v-head) given S (h) and dSn (the chain's dh).
-// [64][128] products: wave w owns row block tb = w % 4 and column blocks
-// 4 (w / 4) .. +3.  [64][64] products: row block ib = w / 2, column blocks
-// 2 (w % 2), +1.  Row and column sums of the dgam / dbeta terms go through
-// per-contributor partial arrays (fixed summation order).
+//
+// Every matrix is held transposed in the accumulators (rows = the contiguous
+// index of the row-major operand, column = token), so a lane's 4 values are
+// 8 adjacent bf16 bytes of one token's row: LDS writes and global stores are
+// packed, and a row sum is an in-lane sum plus two cross-group steps.
+//   P1  K S^T, K dSn^T (wave w: state rows v 16 w .. +15, straight from the
+//       registers S and dSn were loaded into); the lower 16x16 tiles of
+//       Q K^T and K K^T (kept in registers for P3, P to LDS)
+//   P2  X, Vn = Tm X, dVn = P^T dO + Dc K dSn^T, dX = Tm^T dVn, dV, all of
+//       them split along v, so a wave only exchanges data with itself
+//   P3  the lower tiles of dP = dO Vn^T and dA = -dX Vn^T (the inverse's
+//       gradient -Tm^T (dVn X^T) Tm^T with its outer factors applied:
+//       Tm^T dVn = dX, Tm X = Vn), their row and column sums
+//   P4  dQ and dK, wave w: tokens 32 (w % 2) .. +31, columns 32 (w / 2) .. +31
+//
+// What bounds it, at 32 768 tokens qk16/v32 (one workgroup per CU, 151 KB of
+// LDS): a step ((chunk, v-head)) takes about 26 000 cycles, of which the VALU
+// is busy 37%, the LDS 41% and the matrix cores 17%; HBM carries 2.5 GB in
+// 0.72 ms.  It replaces a form that took 1.65 ms with the same products split
+// by rows over 13 barriers per v-head: there Tm was inverted again by one wave
+// of every workgroup, S and dSn were read from HBM twice, and nothing of the
+// next unit was in flight.  The next step's loads go out over P3 and P4,
+// where registers are free: issued together at the top of P4 they held up
+// half of the waves (0.86 ms), issued at P1 they spilled (1.19 ms).
+// Sums over a token's row go through per-contributor partial arrays (fixed
+// summation order).
 struct GradParts {
-  float ag[2][C];    // dgam rows, [64][128] products (contributor w / 4)
-  float ab[2][C];    // dbeta rows, [64][128] products
-  float vk[2][C];    // Dc rowsum(Vn K dSn^T)
-  float tg[2][C];    // dgam rows, [64][64] products (contributor w % 2)
-  float tb[2][C];    // dbeta rows, [64][64] products
-  float tc[4][C];    // dgam column sums (to subtract), [64][64] products (contributor w / 2)
-  float dot[8];      // <dSn, S> per wave
+  float ag[8][C];    // dgam rows of the [64][128] products (contributor: wave)
+  float ab[8][C];    // dbeta rows of the [64][128] products
+  float tg[4][C];    // dgam rows, [64][64] products (contributor: column block)
+  float tb[4][C];    // dbeta rows, [64][64] products
+  float tc[4][C];    // dgam column sums (to subtract), [64][64] products (contributor: row block)
+  float aq[4][C];    // scale E rowsum(Q (dO S)) (contributor: column quarter)
+  float dot[2][8];   // <dSn, S> per wave, by parity of the step
+  float vks[8];      // sum of Dc rowsum(Vn K dSn^T) per wave
 };
 
-template <typename CuT>
+// 4 adjacent bf16 values as floats, and back (round to nearest even).
+__device__ __forceinline__ f32x4 bf4_f32(const uint2& w) {
+  float x0, x1, x2, x3;
+  unpack_bf16x2(w.x, x0, x1);
+  unpack_bf16x2(w.y, x2, x3);
+  return f32x4{x0, x1, x2, x3};
+}
+
+__device__ __forceinline__ void st_bf4(uint16_t* p, const f32x4& x) {
+  *reinterpret_cast<uint2*>(p) = uint2{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3])};
+}
+
+__device__ __forceinline__ bf16x8_t as_bf8(const uint4& w) { return __builtin_bit_cast(bf16x8_t, w); }
+
+// c + x . y for two packed bf16 pairs, in fp32.
+__device__ __forceinline__ float dot2_bf16(uint32_t x, uint32_t y, float c) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, x), __builtin_bit_cast(bf16x2_t, y), c,
+                                         false);
+}
+
+// 4 consecutive values of a gradient row, as fp32 or bf16.
+__device__ __forceinline__ void st_grad(float* p, const f32x4& x) { *reinterpret_cast<f32x4*>(p) = x; }
+__device__ __forceinline__ void st_grad(uint16_t* p, const f32x4& x) { st_bf4(p, x); }
+
+// LDS rows of the gradient kernel: 272 B for [*][128] (the packed 8-byte
+// writes of 16 tokens then hit distinct banks; 288 B, which favours the
+// 16-byte reads instead, is 1% slower), 160 B for [*][64].
+constexpr int GLK = D + 8;
+constexpr int GLC = C + 16;
+
+// What the gate gradients of a training step add (GradT = uint16_t): da, db
+// (bf16, [T, HV]) in place of dg, dbeta, and per (chunk slot, v-head) the
+// terms dg g and da of dA_log and ddt_bias summed over the chunk.
+struct GateOut {
+  void* g;            // dg (fp32) or da (bf16)
+  void* beta;         // dbeta (fp32) or db (bf16)
+  float2* parts;      // [slots][HV], GradT = uint16_t only
+};
+
+template <typename GradT>
 __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const float* __restrict__ A_log, const uint16_t* __restrict__ a, const float* __restrict__ dt_bias,
-    const uint16_t* __restrict__ b, const CuT* __restrict__ cu, int N, int T, int HQ, int HV,
-    float scale, const uint16_t* __restrict__ d_out, const uint16_t* __restrict__ h, int h_chunks,
-    const uint16_t* __restrict__ dh, float* __restrict__ dq, float* __restrict__ dk,
-    float* __restrict__ dv, float* __restrict__ dg, float* __restrict__ dbeta) {
-  __shared__ __align__(16) uint16_t sK_rows[kCB];
-  __shared__ __align__(16) uint16_t sQ_rows[kCB];
-  __shared__ __align__(16) uint16_t sdO[kCB];
-  __shared__ __align__(16) uint16_t sVn[kCB];
-  __shared__ __align__(16) uint16_t sX[kCB];      // V; X; then -beta E dX
-  __shared__ __align__(16) uint16_t sS[2 * kCB];  // dVn | Ar (fp32); then S, dSn [128][LDK]
-  __shared__ __align__(16) uint16_t sTm[kTB];     // Tm; then dPm
-  __shared__ __align__(16) uint16_t sP[kTB];
-  __shared__ __align__(16) uint16_t sdT[kTB];     // dTm; then dAb
-  __shared__ __align__(16) uint16_t sY[kTB];
-  __shared__ __align__(16) float gb[GB_SZ];
+    const uint16_t* __restrict__ b, int HQ, int HV, float scale, const uint16_t* __restrict__ d_out, const uint16_t* __restrict__ h, int h_chunks,
+    int slots, const int2* __restrict__ chunks, const uint16_t* __restrict__ tmrec, const uint16_t* __restrict__ dh,
+    GradT* __restrict__ dq, GradT* __restrict__ dk, GradT* __restrict__ dv, GateOut go) {
+  constexpr bool kStep = std::is_same<GradT, uint16_t>::value;
+  __shared__ __align__(16) uint16_t sK[C * GLK];
+  __shared__ __align__(16) uint16_t sQ[C * GLK];
+  __shared__ __align__(16) uint16_t sdO[C * GLK];
+  __shared__ __align__(16) uint16_t sVn[C * GLK];   // X; then Vn
+  __shared__ __align__(16) uint16_t sdX[C * GLK];   // dVn; then dX
+  __shared__ __align__(16) uint16_t sS[D * GLK];    // S; then dSn
+  __shared__ __align__(16) uint16_t sP[C * GLC];    // P; then dPm
+  __shared__ __align__(16) uint16_t sB[C * GLC];    // Tm; then dAb + dAb^T
+  __shared__ __align__(16) float gbuf[2][GB_SZ + (kStep ? 3 * C : 0)];
   __shared__ GradParts pt;
-  uint16_t* sdV = sS;
-  float* sAr = reinterpret_cast<float*>(sS + kCB);
 
-  int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int g4 = lane >> 4, c16 = lane & 15;
-  // One (chunk, qk-head) per workgroup: its G v-heads in turn, dq and dk
-  // summed over them in registers (v-head order) and stored once.
-  const int slot = blockIdx.x, hq = blockIdx.y;
+  const int tid0 = threadIdx.x, lane0 = tid0 & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
   const int G = HV / HQ;
-  if (slot >= h_chunks) return;
-  int n, ci;
-  locate_chunk(cu, N, T, slot, lane, n, ci);
-  if (n < 0) return;
-  int bos, slen;
-  seq_bounds(cu, n, T, bos, slen);
-  const int t0 = bos + C * ci;
-  const int len = min(C, slen - C * ci);
-  uint4 wk[2], wq[2];
-  rows_fetch(wk, k + size_t(hq) * D, size_t(HQ) * D, t0, len, tid);
-  rows_fetch(wq, q + size_t(hq) * D, size_t(HQ) * D, t0, len, tid);
-  rows_store(sK_rows, wk, tid);
-  rows_store(sQ_rows, wq, tid);
-  const int tb = wave & 3, d0 = 4 * (wave >> 2);
-  const int ib = wave >> 1, j0 = 2 * (wave & 1);
-  f32x4 dq_acc[4], dk_acc[4];     // this wave's dq / dk tiles, summed over the v-heads
-
-  for (int m = 0; m < G; ++m) {
-  // K and Q rows stay in LDS across the v-heads; an offset the compiler
-  // cannot see through (zero) keeps their reads inside the iteration, where
-  // the registers are, instead of hoisted out of the loop.
-  int lds0 = 0;
-  asm volatile("" : "+s"(lds0));
-  uint16_t* sK = sK_rows + lds0;
-  uint16_t* sQ = sQ_rows + lds0;
-  // likewise the lane indices: their address arithmetic is formed where it is used
-  asm volatile("" : "+v"(tid), "+v"(lane), "+v"(g4), "+v"(c16));
-  const int hv = hq * G + m;
-  const size_t rec = (size_t(slot) * HV + hv) * D * D;
-  const uint16_t* Sg = h + rec;
-  const uint16_t* dSg = dh + rec;
-
-  GateIn gi{};
-  if (wave == 0) gi = gate_inputs(A_log, a, dt_bias, b, HV, hv, t0, len, lane);
-  uint4 wo[2], wv[2];
-  rows_fetch(wo, d_out + size_t(hv) * D, size_t(HV) * D, t0, len, tid);
-  rows_fetch(wv, v + size_t(hv) * D, size_t(HV) * D, t0, len, tid);
-  // the previous v-head's last reads of these buffers are behind the barrier
-  // that ends its iteration
-  for (int x = tid; x < C * LDA; x += kGradThreads) sAr[x] = 0.f;
-  for (int x = tid; x < kTB; x += kGradThreads) sP[x] = 0;
-  rows_store(sdO, wo, tid);
-  rows_store(sX, wv, tid);
-  if (wave == 0) chunk_gates_calc(gi, len, lane, gb);
-  lds_barrier();
-
-  ar_p_tiles(sK, sQ, gb, scale, sAr, sP, wave, lane);
-  lds_barrier();
-
-  f32x4 eks[4], xr[4], kds[4];
-  // the inverse's fp32 blocks over sVn, its staging over sY (both unused until later)
-  if (wave == 0) unit_lower_inverse(sAr, gb, reinterpret_cast<float*>(sVn), reinterpret_cast<float*>(sY), sTm, lane);
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int db = d0 + u;
-    f32x4 ks = {0.f, 0.f, 0.f, 0.f}, kd = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s) {
-      const bf16x8_t ko = op_mr(sK, LDK, 16 * tb, 32 * s, lane);
-      ks = mfma16_bf(ko, op_mr(Sg, D, 16 * db, 32 * s, lane), ks);
-      kd = mfma16_bf(ko, op_mr(dSg, D, 16 * db, 32 * s, lane), kd);
+  // Workgroups walk the (chunk slot, qk-head) units, qk-head fastest, and a
+  // unit's G v-heads in turn, dq and dk summed over them in registers (v-head
+  // order).  The next step's rows, states and gate inputs are loaded into
+  // registers while this one is worked on.
+  const int units = slots * HQ;
+  struct At {
+    int unit, m, t0, len;
+  };
+  // the first unit at or after `unit` (in this workgroup's stride) that holds
+  // a chunk; unit >= units when there is none
+  auto seek = [&](int unit) {
+    At x{unit, 0, 0, 0};
+    for (; x.unit < units; x.unit += int(gridDim.x)) {
+      const int slot = x.unit / HQ;
+      if (slot >= h_chunks) continue;
+      const int2 ch = chunks[slot];
+      x.t0 = ch.x;
+      x.len = ch.y;
+      if (ch.y > 0) break;
     }
-    kds[u] = kd;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * tb + 4 * g4 + i;
-      eks[u][i] = gb[GB_E + row] * ks[i];
-      xr[u][i] = bf16_bits_to_f32(sX[row * LDK + 16 * db + c16]) - eks[u][i];
+    return x;
+  };
+  struct Regs {
+    uint4 k[2], q[2], o[2], tm, s[4], ds[4];
+    uint2 v[4];
+  };
+  auto fetch = [&](const At& x, Regs& r, int tid, int lane) {
+    const int slot = x.unit / HQ, hq = x.unit - slot * HQ, hv = hq * G + x.m;
+    const size_t rec = size_t(slot) * HV + hv;
+    if (x.m == 0) {
+      rows_fetch(r.k, k + size_t(hq) * D, size_t(HQ) * D, x.t0, x.len, tid);
+      rows_fetch(r.q, q + size_t(hq) * D, size_t(HQ) * D, x.t0, x.len, tid);
     }
-  }
-  lds_barrier();
+    rows_fetch(r.o, d_out + size_t(hv) * D, size_t(HV) * D, x.t0, x.len, tid);
+    r.tm = reinterpret_cast<const uint4*>(tmrec + rec * C * C)[tid];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    f32x4 x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = gb[GB_BETA + 16 * tb + 4 * g4 + i] * xr[u][i];
-    st_tile(sX, LDK, 16 * tb, 16 * (d0 + u), x, lane);
-  }
-  lds_barrier();
-
-  // Vn = Tm X;  dVn = Dc K dSn^T + P^T dO
-  f32x4 vn[4];
-  float vkp[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int db = d0 + u;
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < C / 32; ++s)
-      x = mfma16_bf(op_mr(sTm, LDC, 16 * tb, 32 * s, lane), op_rm(sX, LDK, 16 * db, 32 * s, lane), x);
-    vn[u] = x;
-    st_tile(sVn, LDK, 16 * tb, 16 * db, x, lane);
-    f32x4 y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      y[i] = gb[GB_DC + 16 * tb + 4 * g4 + i] * kds[u][i];
-      vkp[i] = fmaf(x[i], kds[u][i], vkp[i]);
+    for (int tb = 0; tb < 4; ++tb) {
+      const int t = 16 * tb + (lane & 15);
+      r.v[tb] = t < x.len ? *reinterpret_cast<const uint2*>(v + (size_t(x.t0 + t) * HV + hv) * D +
+                                                            16 * wave + 4 * (lane >> 4))
+                          : uint2{0, 0};
     }
+  };
+  // this wave's 16 rows of a state record (S or dSn) as MFMA operands
+  auto fetch_state = [&](const At& x, const uint16_t* rec0, uint4 (&r)[4], int lane) {
+    const int slot = x.unit / HQ, hv = (x.unit - slot * HQ) * G + x.m;
+    const uint16_t* p = rec0 + (size_t(slot) * HV + hv) * D * D + (16 * wave + (lane & 15)) * D + 8 * (lane >> 4);
 #pragma unroll
-    for (int s = 0; s < C / 32; ++s)
-      y = mfma16_bf(op_rm(sP, LDC, 16 * tb, 32 * s, lane), op_rm(sdO, LDK, 16 * db, 32 * s, lane), y);
-    st_tile(sdV, LDK, 16 * tb, 16 * db, y, lane);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float t = row16_sum(vkp[i]);
-    const int row = 16 * tb + 4 * g4 + i;
-    if (c16 == 0) pt.vk[wave >> 2][row] = gb[GB_DC + row] * t;
-  }
-  lds_barrier();
+    for (int s = 0; s < 4; ++s) r[s] = *reinterpret_cast<const uint4*>(p + 32 * s);
+  };
 
-  // dX = Tm^T dVn (dV, dbeta / dgam terms);  dTm = dVn X^T
-  f32x4 dx[4];
-  float dgr[4] = {0.f, 0.f, 0.f, 0.f}, dbr[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int db = d0 + u;
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < C / 32; ++s)
-      x = mfma16_bf(op_rm(sTm, LDC, 16 * tb, 32 * s, lane), op_rm(sdV, LDK, 16 * db, 32 * s, lane), x);
-    dx[u] = x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * tb + 4 * g4 + i;
-      const float be = gb[GB_BETA + row];
-      dbr[i] = fmaf(x[i], xr[u][i], dbr[i]);
-      dgr[i] = fmaf(-be * x[i], eks[u][i], dgr[i]);
-      if (row < len) dv[(size_t(t0 + row) * HV + hv) * D + 16 * db + c16] = be * x[i];
+  // a step's gate data, formed one step ahead by wave 1
+  auto gate_in = [&](const At& x, int lane) {
+    const int slot = x.unit / HQ;
+    return gate_inputs(A_log, a, dt_bias, b, HV, (x.unit - slot * HQ) * G + x.m, x.t0, x.len, lane);
+  };
+  auto gates = [&](const GateIn& gi, int len, int lane, float* gb) {
+    chunk_gates_calc(gi, len, lane, gb);
+    if constexpr (kStep) {
+      const GateFactors f = gate_factors(gi.a + gi.dt, gi.b, expf(gi.alog));
+      gb[GB_DA + lane] = f.da;
+      gb[GB_DB + lane] = f.db;
+      gb[GB_G + lane] = f.g;
     }
-  }
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s)
-      x = mfma16_bf(op_mr(sdV, LDK, 16 * ib, 32 * s, lane), op_mr(sX, LDK, 16 * (j0 + u), 32 * s, lane), x);
-    st_tile(sdT, LDC, 16 * ib, 16 * (j0 + u), x, lane);
-  }
-  lds_barrier();
+  };
 
-  // -beta E dX -> sX;  Y = dTm Tm^T
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    f32x4 x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * tb + 4 * g4 + i;
-      x[i] = -gb[GB_BETA + row] * gb[GB_E + row] * dx[u][i];
-    }
-    st_tile(sX, LDK, 16 * tb, 16 * (d0 + u), x, lane);
+  // the tiles of sP above the diagonal that an operand read covers stay zero
+  for (int x = tid0; x < 2 * 16 * 16; x += kGradThreads) {
+    const int up = x >> 8, r = (x >> 4) & 15, c = x & 15;
+    sP[(32 * up + r) * GLC + 32 * up + 16 + c] = 0;
   }
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < C / 32; ++s)
-      x = mfma16_bf(op_mr(sdT, LDC, 16 * ib, 32 * s, lane), op_mr(sTm, LDC, 16 * (j0 + u), 32 * s, lane), x);
-    st_tile(sY, LDC, 16 * ib, 16 * (j0 + u), x, lane);
-  }
-  lds_barrier();
 
-  // dA = -Tm^T Y (strictly lower), dP = dO Vn^T (inclusive lower): their dbeta / dgam terms
-  uint4 wst[4];
-  state_fetch(wst, Sg, tid);
-  f32x4 dab[2], dpm[2];
-  {
-    float rg[4] = {0.f, 0.f, 0.f, 0.f}, rb[4] = {0.f, 0.f, 0.f, 0.f};
+  Regs cur;
+  At at = seek(int(blockIdx.x));
+  if (at.unit >= units) return;
+  fetch(at, cur, tid0, lane0);
+  fetch_state(at, h, cur.s, lane0);
+  fetch_state(at, dh, cur.ds, lane0);
+  if (wave == 1) gates(gate_in(at, lane0), at.len, lane0, gbuf[0]);
+  f32x4 dq_acc[2][2], dk_acc[2][2];      // [column block][token block], summed over the v-heads
+  for (int it = 0; at.unit < units; ++it) {
+    // Lane indices opaque to the compiler at the top of each phase: their
+    // address arithmetic is formed where it is used instead of being kept in
+    // registers across phases and steps.
+    int tid = tid0, lane = lane0, g, c;
+    auto fresh_lane = [&] {
+      asm volatile("" : "+v"(lane));
+      g = lane >> 4;
+      c = lane & 15;
+    };
+    asm volatile("" : "+v"(tid));
+    fresh_lane();
+    const int slot = at.unit / HQ, hq = at.unit - slot * HQ, hv = hq * G + at.m;
+    const int t0 = at.t0, len = at.len, m = at.m;
+    float* gb = gbuf[it & 1];
+
+    // P0: rows to LDS
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int jb = j0 + u;
-      f32x4 da = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < C / 32; ++s)
-        da = mfma16_bf(op_rm(sTm, LDC, 16 * ib, 32 * s, lane), op_rm(sY, LDC, 16 * jb, 32 * s, lane), da);
-#pragma unroll
-      for (int s = 0; s < D / 32; ++s)
-        dp = mfma16_bf(op_mr(sdO, LDK, 16 * ib, 32 * s, lane), op_mr(sVn, LDK, 16 * jb, 32 * s, lane), dp);
-      const int col = 16 * jb + c16;
-      const float gc = gb[GB_GAM + col];
-      float cs = 0.f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 16 * ib + 4 * g4 + i;
-        const float ex = row >= col ? expf(gb[GB_GAM + row] - gc) : 0.f;
-        const float dA = row > col ? -da[i] : 0.f;
-        const float dP = row >= col ? dp[i] : 0.f;
-        const float ar = sAr[row * LDA + col];
-        const float be = gb[GB_BETA + row];
-        const float pv = bf16_bits_to_f32(sP[row * LDC + col]);
-        const float aa = dA * be * ar, pp = dP * pv;
-        rb[i] = fmaf(dA, ar, rb[i]);
-        rg[i] += aa + pp;
-        cs += aa + pp;
-        dab[u][i] = be * ex * dA;
-        dpm[u][i] = scale * ex * dP;
+    for (int i = 0; i < 2; ++i) {
+      const int x = tid + i * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
+      if (m == 0) {
+        *reinterpret_cast<uint4*>(sK + r * GLK + cc) = cur.k[i];
+        *reinterpret_cast<uint4*>(sQ + r * GLK + cc) = cur.q[i];
       }
-      cs = group4_sum(cs);
-      if (g4 == 0) pt.tc[ib][col] = cs;
+      *reinterpret_cast<uint4*>(sdO + r * GLK + cc) = cur.o[i];
     }
+    *reinterpret_cast<uint4*>(sB + (tid >> 3) * GLC + 8 * (tid & 7)) = cur.tm;
+    lds_barrier();
+
+    // P1: K S^T and K dSn^T, transposed: rows v = 16 wave + 4 g + i, column t = 16 tb + c
+    f32x4 ks[4], kd[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float tg = row16_sum(rg[i]), tbv = row16_sum(rb[i]);
-      const int row = 16 * ib + 4 * g4 + i;
-      if (c16 == 0) {
-        pt.tg[wave & 1][row] = tg;
-        pt.tb[wave & 1][row] = tbv;
+    for (int tb = 0; tb < 4; ++tb) {
+      ks[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      kd[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bf16x8_t ko = op_mr(sK, GLK, 16 * tb, 32 * s, lane);
+        ks[tb] = mfma16_bf(as_bf8(cur.s[s]), ko, ks[tb]);
+        kd[tb] = mfma16_bf(as_bf8(cur.ds[s]), ko, kd[tb]);
       }
     }
-  }
-  lds_barrier();
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    st_tile(sdT, LDC, 16 * ib, 16 * (j0 + u), dab[u], lane);
-    st_tile(sTm, LDC, 16 * ib, 16 * (j0 + u), dpm[u], lane);
-  }
-  // S -> LDS [v][LDK] over dVn and Ar (both read for the last time above)
-  state_store(sS, wst, tid);
-  lds_barrier();
-
-  // dQ = scale E dO S + dPm K;  dK (all but the dSn term) = -beta E dX S + dPm^T Q + dAb K + dAb^T K
-  uint4 wds[4];
-  state_fetch(wds, dSg, tid);
-  f32x4 dkp[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int kb = d0 + u;
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s)
-      x = mfma16_bf(op_mr(sdO, LDK, 16 * tb, 32 * s, lane), op_rm(sS, LDK, 16 * kb, 32 * s, lane), x);
-    f32x4 y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * tb + 4 * g4 + i;
-      y[i] = scale * gb[GB_E + row] * x[i];
-      dgr[i] = fmaf(y[i], bf16_bits_to_f32(sQ[row * LDK + 16 * kb + c16]), dgr[i]);
-    }
-#pragma unroll
-    for (int s = 0; s < C / 32; ++s)
-      y = mfma16_bf(op_mr(sTm, LDC, 16 * tb, 32 * s, lane), op_rm(sK, LDK, 16 * kb, 32 * s, lane), y);
-    if (m == 0) dq_acc[u] = y;
-    else dq_acc[u] += y;
-    f32x4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s)
-      z = mfma16_bf(op_mr(sX, LDK, 16 * tb, 32 * s, lane), op_rm(sS, LDK, 16 * kb, 32 * s, lane), z);
-#pragma unroll
-    for (int s = 0; s < C / 32; ++s) {
-      const bf16x8_t kop = op_rm(sK, LDK, 16 * kb, 32 * s, lane);
-      z = mfma16_bf(op_rm(sTm, LDC, 16 * tb, 32 * s, lane), op_rm(sQ, LDK, 16 * kb, 32 * s, lane), z);
-      z = mfma16_bf(op_mr(sdT, LDC, 16 * tb, 32 * s, lane), kop, z);
-      z = mfma16_bf(op_rm(sdT, LDC, 16 * tb, 32 * s, lane), kop, z);
-    }
-    dkp[u] = z;
-  }
-  {
-    // <dSn, S>: this thread's 32 elements of S (in LDS) against those of dSn
-    float part = 0.f;
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int x = tid + it * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
-      const uint4 sw = *reinterpret_cast<const uint4*>(&sS[r * LDK + cc]);
-      const uint32_t ss[4] = {sw.x, sw.y, sw.z, sw.w};
-      const uint32_t dd[4] = {wds[it].x, wds[it].y, wds[it].z, wds[it].w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float s0, s1, d0, d1;
-        unpack_bf16x2(ss[j], s0, s1);
-        unpack_bf16x2(dd[j], d0, d1);
-        part = fmaf(s0, d0, fmaf(s1, d1, part));
-      }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off);
-    if (lane == 0) pt.dot[wave] = part;
-  }
-  lds_barrier();
-  state_store(sS, wds, tid);
-  lds_barrier();
-
-  // dK += Dc Vn dSn
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int kb = d0 + u;
-    f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < D / 32; ++s)
-      x = mfma16_bf(op_mr(sVn, LDK, 16 * tb, 32 * s, lane), op_rm(sS, LDK, 16 * kb, 32 * s, lane), x);
-    f32x4 z;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) z[i] = fmaf(gb[GB_DC + 16 * tb + 4 * g4 + i], x[i], dkp[u][i]);
-    if (m == 0) dk_acc[u] = z;
-    else dk_acc[u] += z;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float tg = row16_sum(dgr[i]), tbv = row16_sum(dbr[i]);
-    const int row = 16 * tb + 4 * g4 + i;
-    if (c16 == 0) {
-      pt.ag[wave >> 2][row] = tg;
-      pt.ab[wave >> 2][row] = tbv;
-    }
-  }
-  lds_barrier();
-
-  if (wave == 0) {
-    const int t = lane;
-    const float vk = pt.vk[0][t] + pt.vk[1][t];
-    float dgam = pt.ag[0][t] + pt.ag[1][t] - vk + pt.tg[0][t] + pt.tg[1][t] -
-                 ((pt.tc[0][t] + pt.tc[1][t]) + (pt.tc[2][t] + pt.tc[3][t]));
-    float vks = vk;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) vks += __shfl_xor(vks, off);
     float dot = 0.f;
 #pragma unroll
-    for (int w = 0; w < 8; ++w) dot += pt.dot[w];
-    if (t == C - 1) dgam += vks + gb[GB_EL] * dot;
-    // dg_t = sum_{i >= t} dgam_i
-    const float incl = wave_inclusive_scan(dgam);
-    const float total = __shfl(incl, 63);
-    const float dgt = total - incl + dgam;
-    const float dbt = (pt.ab[0][t] + pt.ab[1][t]) + (pt.tb[0][t] + pt.tb[1][t]);
-    if (t < len) {
-      dg[size_t(t0 + t) * HV + hv] = dgt;
-      dbeta[size_t(t0 + t) * HV + hv] = dbt;
+    for (int s = 0; s < 4; ++s) {
+      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * GLK + 32 * s + 8 * g) = cur.s[s];
+      const uint32_t ss[4] = {cur.s[s].x, cur.s[s].y, cur.s[s].z, cur.s[s].w};
+      const uint32_t dd[4] = {cur.ds[s].x, cur.ds[s].y, cur.ds[s].z, cur.ds[s].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dot = dot2_bf16(ss[j], dd[j], dot);
     }
-  }
-  lds_barrier();    // the next v-head rewrites every buffer but sK, sQ
-  }
+    // tiles (ti, tj) of Q K^T and K K^T: wave w takes tile w, waves 6 and 7 also 8 and 9
+    f32x4 qk[2], kk[2], ex[2];
+    auto tile_of = [&](int j, int& ti, int& tj) {
+      const int tile = wave + 2 * j;
+      ti = tile < 1 ? 0 : tile < 3 ? 1 : tile < 6 ? 2 : 3;
+      tj = tile - (ti * (ti + 1)) / 2;
+    };
+    auto qk_tiles = [&](auto count) {
+      constexpr int n = decltype(count)::value;
+#pragma unroll
+      for (int j = 0; j < n; ++j) qk[j] = kk[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < n; ++j) {
+          int ti, tj;
+          tile_of(j, ti, tj);
+          const bf16x8_t ka = op_mr(sK, GLK, 16 * tj, 32 * s, lane);
+          qk[j] = mfma16_bf(ka, op_mr(sQ, GLK, 16 * ti, 32 * s, lane), qk[j]);
+          kk[j] = mfma16_bf(ka, op_mr(sK, GLK, 16 * ti, 32 * s, lane), kk[j]);
+        }
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        int ti, tj;
+        tile_of(j, ti, tj);
+        const int t = 16 * ti + c, s0 = 16 * tj + 4 * g;
+        const float gt = gb[GB_GAM + t];
+        const f32x4 gs = *reinterpret_cast<const f32x4*>(&gb[GB_GAM + s0]);
+        f32x4 pv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ex[j][i] = t >= s0 + i ? exp_fast(gt - gs[i]) : 0.f;
+          pv[i] = scale * (ex[j][i] * qk[j][i]);
+        }
+        st_bf4(sP + t * GLC + s0, pv);
+      }
+    };
+    if (wave >= 6) qk_tiles(IC<2>());
+    else qk_tiles(IC<1>());
+    dot = wave_inclusive_scan(dot);
+    if (lane == 63) pt.dot[it & 1][wave] = dot;
+    At nx = at;
+    ++nx.m;
+    if (nx.m == G) nx = seek(at.unit + int(gridDim.x));
+    const bool more = nx.unit < units;
+    GateIn gin{};
+    if (wave == 1 && more) gin = gate_in(nx, lane);
+    lds_barrier();
 
+    // P2: everything split along v (this wave's 16 rows of the transposed tiles)
+    fresh_lane();
+    {
+      const int v0 = 16 * wave + 4 * g;     // first of this lane's 4 columns v
+      f32x4 xr[4], vn[4], dx[4];
+      bf16x8_t xo[2], yo[2];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+      for (int s = 0; s < 2; ++s) yo[s] = op_rm(sdO, GLK, 16 * wave, 32 * s, lane);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = 16 * tb + 4 * g4 + i;
-      if (row < len) {
-        const size_t at = (size_t(t0 + row) * HQ + hq) * D + 16 * (d0 + u) + c16;
-        dq[at] = dq_acc[u][i];
-        dk[at] = dk_acc[u][i];
+      for (int tb = 0; tb < 4; ++tb) {
+        const int t = 16 * tb + c;
+        const float e = gb[GB_E + t], be = gb[GB_BETA + t], dc = gb[GB_DC + t];
+        const f32x4 vv = bf4_f32(cur.v[tb]);
+        f32x4 x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          ks[tb][i] *= e;
+          xr[tb][i] = vv[i] - ks[tb][i];
+          x[i] = be * xr[tb][i];
+          kd[tb][i] *= dc;
+        }
+        st_bf4(sVn + t * GLK + v0, x);
+        // dVn = Dc K dSn^T + P^T dO
+        dx[tb] = kd[tb];
+#pragma unroll
+        for (int s = tb / 2; s < 2; ++s)
+          dx[tb] = mfma16_bf(yo[s], op_rm(sP, GLC, 16 * tb, 32 * s, lane), dx[tb]);
+        st_bf4(sdX + t * GLK + v0, dx[tb]);
+      }
+      // Vn = Tm X and dX = Tm^T dVn (Tm lower: rows 0-31 of Tm need only their
+      // own 32 columns, rows 32-63 of Tm^T likewise)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        xo[s] = op_rm(sVn, GLK, 16 * wave, 32 * s, lane);
+        yo[s] = op_rm(sdX, GLK, 16 * wave, 32 * s, lane);
+      }
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) {
+        vn[tb] = dx[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (s <= tb / 2) vn[tb] = mfma16_bf(xo[s], op_mr(sB, GLC, 16 * tb, 32 * s, lane), vn[tb]);
+          if (s >= tb / 2) dx[tb] = mfma16_bf(yo[s], op_rm(sB, GLC, 16 * tb, 32 * s, lane), dx[tb]);
+        }
+      }
+      float vks = 0.f;
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) {
+        const int t = 16 * tb + c;
+        const float be = gb[GB_BETA + t];
+        st_bf4(sVn + t * GLK + v0, vn[tb]);
+        st_bf4(sdX + t * GLK + v0, dx[tb]);
+        f32x4 dvv;
+        float sg = 0.f, sb = 0.f, sv = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          dvv[i] = be * dx[tb][i];
+          sb = fmaf(dx[tb][i], xr[tb][i], sb);
+          sg = fmaf(dvv[i], ks[tb][i], sg);
+          sv = fmaf(vn[tb][i], kd[tb][i], sv);
+        }
+        if (t < len) st_grad(dv + (size_t(t0 + t) * HV + hv) * D + v0, dvv);
+        vks += sv;
+        sg = group4_sum(-sg - sv);
+        sb = group4_sum(sb);
+        if (g == 0) {
+          pt.ag[wave][t] = sg;
+          pt.ab[wave][t] = sb;
+        }
+      }
+      vks = wave_inclusive_scan(vks);
+      if (lane == 63) pt.vks[wave] = vks;
+    }
+    lds_barrier();
+
+    fresh_lane();
+    // the next step's inputs are loaded over P3 and P4
+    Regs nxt;
+    if (more) fetch(nx, nxt, tid, lane);
+    // P3: dP and dA tiles (rows s = 16 tj + 4 g + i, column t = 16 ti + c)
+    auto da_tiles = [&](auto count) {
+      constexpr int n = decltype(count)::value;
+      f32x4 dp[n], da[n];
+#pragma unroll
+      for (int j = 0; j < n; ++j) dp[j] = da[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < n; ++j) {
+          int ti, tj;
+          tile_of(j, ti, tj);
+          const bf16x8_t va = op_mr(sVn, GLK, 16 * tj, 32 * s, lane);
+          dp[j] = mfma16_bf(va, op_mr(sdO, GLK, 16 * ti, 32 * s, lane), dp[j]);
+          da[j] = mfma16_bf(va, op_mr(sdX, GLK, 16 * ti, 32 * s, lane), da[j]);
+        }
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        int ti, tj;
+        tile_of(j, ti, tj);
+        const int t = 16 * ti + c, s0 = 16 * tj + 4 * g;
+        const float be = gb[GB_BETA + t];
+        f32x4 dpm, dab, cs;
+        float rg = 0.f, rb = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // ex is zero above the diagonal
+          dpm[i] = scale * ex[j][i] * dp[j][i];
+          const float xa = t > s0 + i ? -ex[j][i] * da[j][i] : 0.f;
+          dab[i] = be * xa;
+          cs[i] = fmaf(dpm[i], qk[j][i], dab[i] * kk[j][i]);
+          rg += cs[i];
+          rb = fmaf(xa, kk[j][i], rb);
+        }
+        st_bf4(sP + t * GLC + s0, dpm);
+        const uint32_t b01 = cvt_pk_bf16(dab[0], dab[1]), b23 = cvt_pk_bf16(dab[2], dab[3]);
+        const uint16_t bb[4] = {uint16_t(b01), uint16_t(b01 >> 16), uint16_t(b23), uint16_t(b23 >> 16)};
+        if (ti != tj) {
+          *reinterpret_cast<uint2*>(sB + t * GLC + s0) = uint2{b01, b23};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sB[(s0 + i) * GLC + t] = bb[i];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (t >= s0 + i) {                // dab is zero on the diagonal
+              sB[t * GLC + s0 + i] = bb[i];
+              sB[(s0 + i) * GLC + t] = bb[i];
+            }
+        }
+        rg = group4_sum(rg);
+        rb = group4_sum(rb);
+        if (g == 0) {
+          pt.tg[tj][t] = rg;
+          pt.tb[tj][t] = rb;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float x = row16_sum(cs[i]);
+          if (c == 0) pt.tc[ti][s0 + i] = x;
+        }
+      }
+    };
+    if (wave >= 6) da_tiles(IC<2>());
+    else da_tiles(IC<1>());
+    if (wave == 1 && more) gates(gin, nx.len, lane, gbuf[(it + 1) & 1]);
+    lds_barrier();
+    if (more) fetch_state(nx, h, nxt.s, lane);
+    // P4: dQ = scale E dO S + dPm K;  dK = Dc Vn dSn - beta E dX S + dPm^T Q + (dAb + dAb^T) K
+    fresh_lane();
+    const int tr0 = 32 * (wave & 1), k0 = 32 * (wave >> 1);
+    f32x4 y[2][2], z[2][2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb) y[kb][tb] = z[kb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      bf16x8_t so[2], oo[2], xo[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        so[u] = op_rm(sS, GLK, k0 + 16 * u, 32 * s, lane);
+        oo[u] = op_mr(sdO, GLK, tr0 + 16 * u, 32 * s, lane);
+        xo[u] = op_mr(sdX, GLK, tr0 + 16 * u, 32 * s, lane);
+      }
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) {
+          y[kb][tb] = mfma16_bf(so[kb], oo[tb], y[kb][tb]);
+          z[kb][tb] = mfma16_bf(so[kb], xo[tb], z[kb][tb]);
+        }
+    }
+    const float e0 = gb[GB_E + tr0 + c], e1 = gb[GB_E + tr0 + 16 + c];
+    const float be0 = gb[GB_BETA + tr0 + c], be1 = gb[GB_BETA + tr0 + 16 + c];
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb) {
+      const int t = tr0 + 16 * tb + c;
+      const float fq = scale * (tb ? e1 : e0), fx = -(tb ? be1 * e1 : be0 * e0);
+      float sq = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const f32x4 qv = bf4_f32(*reinterpret_cast<const uint2*>(sQ + t * GLK + k0 + 16 * kb + 4 * g));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          y[kb][tb][i] *= fq;
+          z[kb][tb][i] *= fx;
+          sq = fmaf(y[kb][tb][i], qv[i], sq);
+        }
+      }
+      sq = group4_sum(sq);
+      if (g == 0) pt.aq[wave >> 1][t] = sq;
+    }
+    // the triangular products: dPm's rows 0-31 end at column 31, dPm^T's rows 32-63 begin at 32
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8_t ko[2], qo[2], po[2], pto[2], bo[2];
+      const bool lo = s == 0 || tr0 != 0, hi = s == 1 || tr0 == 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        ko[u] = op_rm(sK, GLK, k0 + 16 * u, 32 * s, lane);
+        bo[u] = op_mr(sB, GLC, tr0 + 16 * u, 32 * s, lane);
+      }
+      if (lo) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) po[u] = op_mr(sP, GLC, tr0 + 16 * u, 32 * s, lane);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb) y[kb][tb] = mfma16_bf(ko[kb], po[tb], y[kb][tb]);
+      }
+      if (hi) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          qo[u] = op_rm(sQ, GLK, k0 + 16 * u, 32 * s, lane);
+          pto[u] = op_rm(sP, GLC, tr0 + 16 * u, 32 * s, lane);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb) z[kb][tb] = mfma16_bf(qo[kb], pto[tb], z[kb][tb]);
+      }
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) z[kb][tb] = mfma16_bf(ko[kb], bo[tb], z[kb][tb]);
+    }
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * GLK + 32 * s + 8 * g) = cur.ds[s];
+    if (more) fetch_state(nx, dh, nxt.ds, lane);
+    lds_barrier();
+    fresh_lane();
+    {
+      f32x4 x[2][2];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int tb = 0; tb < 2; ++tb) x[kb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        bf16x8_t so[2], vo[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          so[u] = op_rm(sS, GLK, k0 + 16 * u, 32 * s, lane);
+          vo[u] = op_mr(sVn, GLK, tr0 + 16 * u, 32 * s, lane);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int tb = 0; tb < 2; ++tb) x[kb][tb] = mfma16_bf(so[kb], vo[tb], x[kb][tb]);
+      }
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb) {
+        const float dc = gb[GB_DC + tr0 + 16 * tb + c];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) z[kb][tb][i] = fmaf(dc, x[kb][tb][i], z[kb][tb][i]);
+          dq_acc[kb][tb] = m == 0 ? y[kb][tb] : dq_acc[kb][tb] + y[kb][tb];
+          dk_acc[kb][tb] = m == 0 ? z[kb][tb] : dk_acc[kb][tb] + z[kb][tb];
+        }
       }
     }
+    if (m == G - 1) {
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb) {
+        const int t = tr0 + 16 * tb + c;
+        if (t < len) {
+          const size_t row = (size_t(t0 + t) * HQ + hq) * D + k0 + 4 * g;
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb) {
+            st_grad(dq + row + 16 * kb, dq_acc[kb][tb]);
+            st_grad(dk + row + 16 * kb, dk_acc[kb][tb]);
+          }
+        }
+      }
+    }
+    if (wave == 0) {
+      const int t = lane, blk = lane >> 4;
+      float dgam = 0.f, dbt = 0.f, dsum = 0.f, vks = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) {
+        dgam += pt.ag[w][t];
+        dbt += pt.ab[w][t];
+        dsum += pt.dot[it & 1][w];
+        vks += pt.vks[w];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        dgam += pt.aq[j][t];
+        if (j <= blk) {
+          dgam += pt.tg[j][t];
+          dbt += pt.tb[j][t];
+        }
+        if (j >= blk) dgam -= pt.tc[j][t];
+      }
+      if (t == C - 1) dgam += vks + gb[GB_EL] * dsum;
+      // dg_t = sum_{i >= t} dgam_i
+      const float incl = wave_inclusive_scan(dgam);
+      const float total = __shfl(incl, 63);
+      const float dgt = total - incl + dgam;
+      const size_t i = size_t(t0 + t) * HV + hv;
+      if constexpr (kStep) {
+        float sa = 0.f, sd = 0.f;
+        if (t < len) {
+          const float dai = dgt * gb[GB_DA + t], dbi = dbt * gb[GB_DB + t];
+          sa = dgt * gb[GB_G + t];
+          sd = dai;
+          reinterpret_cast<uint16_t*>(go.g)[i] = f32_to_bf16_bits(dai);
+          reinterpret_cast<uint16_t*>(go.beta)[i] = f32_to_bf16_bits(dbi);
+        }
+        sa = wave_inclusive_scan(sa);
+        sd = wave_inclusive_scan(sd);
+        if (lane == 63) go.parts[size_t(slot) * HV + hv] = float2{sa, sd};
+      } else if (t < len) {
+        reinterpret_cast<float*>(go.g)[i] = dgt;
+        reinterpret_cast<float*>(go.beta)[i] = dbt;
+      }
+    }
+    cur = nxt;
+    at = nx;
+  }
 }
 
-// Gradients of the gating, per v-head (one workgroup each):
-//   g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b)
-//   da = dg (-exp(A_log) sigmoid(a + dt_bias)),  ddt_bias = sum_t da,
-//   dA_log = sum_t dg g,  db = dbeta beta (1 - beta).
+// Gradients of the gating, per v-head (one workgroup each), over all tokens.
 __global__ __launch_bounds__(256) void gdn_gate_bwd_kernel(
     const float* __restrict__ A_log, const uint16_t* __restrict__ a, const float* __restrict__ dt_bias,
     const uint16_t* __restrict__ b, const float* __restrict__ dg, const float* __restrict__ dbeta, int T,
@@ -1014,80 +1269,132 @@ __global__ __launch_bounds__(256) void gdn_gate_bwd_kernel(
   float sa = 0.f, sd = 0.f;
   for (int t = tid; t < T; t += 256) {
     const size_t i = size_t(t) * HV + hv;
-    const float x = bf16_bits_to_f32(a[i]) + bias;
-    const float g = dg[i];
-    const float dai = -g * ea * sigmoidf_(x);
-    const float be = sigmoidf_(bf16_bits_to_f32(b[i]));
+    const GateFactors f = gate_factors(bf16_bits_to_f32(a[i]) + bias, bf16_bits_to_f32(b[i]), ea);
+    const float dai = dg[i] * f.da;
     da[i] = dai;
-    db[i] = dbeta[i] * be * (1.f - be);
-    sa = fmaf(g, -ea * softplus_stable(x), sa);
+    db[i] = dbeta[i] * f.db;
+    sa = fmaf(dg[i], f.g, sa);
     sd += dai;
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    sa += __shfl_xor(sa, off);
-    sd += __shfl_xor(sd, off);
-  }
-  if ((tid & 63) == 0) {
-    red[0][tid >> 6] = sa;
-    red[1][tid >> 6] = sd;
-  }
-  __syncthreads();
+  sum_pair_256(sa, sd, red);
   if (tid == 0) {
-    dA_log[hv] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-    ddt_bias[hv] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    dA_log[hv] = sa;
+    ddt_bias[hv] = sd;
   }
 }
 
+// dA_log and ddt_bias of a training step: the chunks' partial sums per v-head
+// (one workgroup each), chunks in a fixed order.
 template <typename CuT>
+__global__ __launch_bounds__(256) void gdn_gate_sums_kernel(const CuT* __restrict__ cu, int N, int T,
+                                                            int HV, int h_chunks,
+                                                            const float2* __restrict__ parts,
+                                                            float* __restrict__ dA_log,
+                                                            float* __restrict__ ddt_bias) {
+  __shared__ float red[2][4];
+  const int hv = blockIdx.x, tid = threadIdx.x;
+  const int chunks = min(h_chunks, chunk_offset(cu, N, T, tid & 63));
+  float sa = 0.f, sd = 0.f;
+  for (int s = tid; s < chunks; s += 256) {
+    const float2 x = parts[size_t(s) * HV + hv];
+    sa += x.x;
+    sd += x.y;
+  }
+  sum_pair_256(sa, sd, red);
+  if (tid == 0) {
+    dA_log[hv] = sa;
+    ddt_bias[hv] = sd;
+  }
+}
+
+// Workspace of a backward over `slots` chunk slots.
+struct BwdWorkspace {
+  char* m;
+  char* r;           // R; the chain kernel leaves dSn there
+  uint16_t* tm;
+  int2* chunks;      // first token and length of every chunk slot (length 0: none)
+  float2* parts;     // over m, which the chain kernel has consumed by then
+  BwdWorkspace(char* ws, size_t slots, size_t HV) {
+    const size_t units = slots * HV;
+    m = ws;
+    r = m + units * kMBytes;
+    tm = reinterpret_cast<uint16_t*>(r + units * kRBytes);
+    chunks = reinterpret_cast<int2*>(tm + units * (kTmBytes / 2));
+    parts = reinterpret_cast<float2*>(m);
+  }
+  static size_t bytes(size_t slots, size_t HV) {
+    return slots * HV * (kMBytes + kRBytes + kTmBytes) + slots * sizeof(int2);
+  }
+};
+
+// GradT = float: fp32 gradients, dg and dbeta in g_out and beta_out.
+// GradT = uint16_t: a training step's, in bf16, with da and db there and the
+// per-head sums in dA_log and ddt_bias.
+template <typename CuT, typename GradT>
 int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* A_log,
                const uint16_t* a, const float* dt_bias, const uint16_t* b, const CuT* cu, int N, int T,
                int HQ, int HV, float scale, const uint16_t* h, int h_chunks, const uint16_t* d_out,
-               const float* d_ht, float* dq, float* dk, float* dv, float* dg, float* dbeta, float* dh0,
-               char* ws, hipStream_t st) {
+               const float* d_ht, GradT* dq, GradT* dk, GradT* dv, GradT* g_out, GradT* beta_out,
+               float* dA_log, float* ddt_bias, float* dh0, char* ws, hipStream_t st) {
   const size_t slots = size_t(T) / C + size_t(N);
   // The workspace holds `slots` chunk records per v-head.  Well-formed
   // cu_seqlens give at most that many chunks; with overlapping ranges the
   // chunk count (and h_chunks) can exceed it, and every kernel then stops at
   // the last slot the workspace holds (results unspecified, accesses in bounds).
   h_chunks = int(std::min<size_t>(size_t(h_chunks), slots));
-  char* mrec = ws;
-  char* rrec = mrec + slots * HV * kMBytes;
-  uint16_t* dhr = reinterpret_cast<uint16_t*>(rrec + slots * HV * kRBytes);
-  // Persistent workgroups, one per CU, when each takes many units (the next
-  // unit's inputs are then fetched during the current one); with few units
-  // per CU, one workgroup per unit, which the dispatcher balances.
-  const int cus = device_cus();
   const size_t units = slots * size_t(HV);
+  const BwdWorkspace w(ws, slots, size_t(HV));
+  const int cus = device_cus();
   const size_t wgs = size_t(cus > 0 ? cus : 256);
-  const unsigned pgrid = unsigned(units >= 8 * wgs ? wgs : units);
-  hipLaunchKernelGGL((gdn_bwd_prep_kernel<CuT>), dim3(pgrid), dim3(kGradThreads), 0, st, q, k, A_log, a,
-                     dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h_chunks, int(slots), mrec, rrec);
-  // The reverse chain: one workgroup of 8 waves per chain, or, when the
-  // chains leave most CUs idle, 4 workgroups of 2 waves (32 state rows) each.
-  const unsigned chain_ids = 8u * ((unsigned(N) * unsigned(HV) + 7u) / 8u);
-  if (cus > 0 && 4LL * N * HV <= cus)
-    hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 2>), dim3(4u * chain_ids), dim3(128), 0, st, cu, N, T,
-                       HV, h_chunks, mrec, rrec, d_ht, dhr, dh0);
-  else
-    hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 8>), dim3(chain_ids), dim3(512), 0, st, cu, N, T, HV,
-                       h_chunks, mrec, rrec, d_ht, dhr, dh0);
-  if (T > 0) {
-    // one workgroup per (chunk, qk-head), its v-heads in turn
-    const dim3 qgrid{unsigned(slots), unsigned(HQ), 1u};
-    hipLaunchKernelGGL((gdn_bwd_grad_kernel<CuT>), qgrid, dim3(kGradThreads), 0, st, q, k, v, A_log, a,
-                       dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h, h_chunks, dhr, dq, dk, dv, dg, dbeta);
+  if (N > 0) {
+    // Persistent workgroups, one per CU, when each takes many units (the next
+    // unit's inputs are then fetched during the current one); with few units
+    // per CU, one workgroup per unit, which the dispatcher balances.
+    const unsigned pgrid = unsigned(units >= 8 * wgs ? wgs : units);
+    hipLaunchKernelGGL((gdn_bwd_prep_kernel<CuT>), dim3(pgrid), dim3(kGradThreads), 0, st, q, k, A_log, a,
+                       dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h_chunks, int(slots), w.m, w.r, w.tm, w.chunks);
+    // The reverse chain: one workgroup of 8 waves per chain, or, when the
+    // chains leave most CUs idle, 4 workgroups of 2 waves (32 state rows) each.
+    const unsigned chain_ids = 8u * ((unsigned(N) * unsigned(HV) + 7u) / 8u);
+    if (cus > 0 && 4LL * N * HV <= cus)
+      hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 2>), dim3(4u * chain_ids), dim3(128), 0, st, cu, N, T,
+                         HV, h_chunks, w.m, w.r, d_ht, dh0);
+    else
+      hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 8>), dim3(chain_ids), dim3(512), 0, st, cu, N, T, HV,
+                         h_chunks, w.m, w.r, d_ht, dh0);
+    if (T > 0) {
+      // one workgroup per CU walks the (chunk, qk-head) units
+      const unsigned ggrid = unsigned(std::min(slots * size_t(HQ), wgs));
+      hipLaunchKernelGGL((gdn_bwd_grad_kernel<GradT>), dim3(ggrid), dim3(kGradThreads), 0, st, q, k, v,
+                         A_log, a, dt_bias, b, HQ, HV, scale, d_out, h, h_chunks, int(slots), w.chunks,
+                         w.tm, reinterpret_cast<const uint16_t*>(w.r), dq, dk, dv,
+                         GateOut{g_out, beta_out, w.parts});
+    }
   }
+  if (dA_log)
+    hipLaunchKernelGGL((gdn_gate_sums_kernel<CuT>), dim3(unsigned(HV)), dim3(256), 0, st, cu, N, T, HV,
+                       h_chunks, w.parts, dA_log, ddt_bias);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? GDN_OK : -int(e);
+}
+
+// The argument checks of both entry points (outputs apart).
+int check_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* A_log, const uint16_t* a,
+              const float* dt_bias, const uint16_t* b, const void* cu, int N, int T, int HQ, int HV,
+              const uint16_t* h, int h_chunks, const uint16_t* d_out, bool outputs) {
+  if (N < 0 || T < 0 || HQ <= 0 || HV <= 0 || HV % HQ != 0 || h_chunks < 0) return GDN_ERR_SHAPE;
+  if (!cu) return GDN_ERR_NULL;
+  if (N > 0 && (!A_log || !dt_bias)) return GDN_ERR_NULL;
+  if (T > 0 && (!q || !k || !v || !a || !b || !d_out || !outputs)) return GDN_ERR_NULL;
+  if (h_chunks > 0 && !h) return GDN_ERR_NULL;
+  return GDN_OK;
 }
 
 }  // namespace
 
 extern "C" size_t gdn_prefill_bwd_workspace_bytes(int N, int T, int HQ, int HV) {
   if (N < 0 || T < 0 || HQ <= 0 || HV <= 0 || HV % HQ != 0) return 0;
-  const size_t slots = size_t(T) / C + size_t(N);
-  return slots * size_t(HV) * (kMBytes + kRBytes + kHBytes);
+  return BwdWorkspace::bytes(size_t(T) / C + size_t(N), size_t(HV));
 }
 
 extern "C" int gdn_prefill_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v,
@@ -1097,24 +1404,44 @@ extern "C" int gdn_prefill_bwd(const uint16_t* q, const uint16_t* k, const uint1
                                const uint16_t* d_out, const float* d_final_state, float* dq, float* dk,
                                float* dv, float* dg, float* dbeta, float* d_initial_state,
                                void* workspace, size_t workspace_bytes, void* stream) {
-  if (N < 0 || T < 0 || HQ <= 0 || HV <= 0 || HV % HQ != 0 || h_chunks < 0) return GDN_ERR_SHAPE;
-  if (!cu_seqlens) return GDN_ERR_NULL;
-  if (N > 0 && (!A_log || !dt_bias)) return GDN_ERR_NULL;
-  if (T > 0 && (!q || !k || !v || !a || !b || !d_out || !dq || !dk || !dv || !dg || !dbeta))
-    return GDN_ERR_NULL;
-  if (h_chunks > 0 && !h) return GDN_ERR_NULL;
-  if (N == 0) return GDN_OK;
+  const int rc = check_bwd(q, k, v, A_log, a, dt_bias, b, cu_seqlens, N, T, HQ, HV, h, h_chunks, d_out,
+                           dq && dk && dv && dg && dbeta);
+  if (rc != GDN_OK || N == 0) return rc;
   if (!workspace || workspace_bytes < gdn_prefill_bwd_workspace_bytes(N, T, HQ, HV))
     return GDN_ERR_WORKSPACE;
   hipStream_t st = static_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
-  if (cu_is_int32)
-    return launch_bwd(q, k, v, A_log, a, dt_bias, b, static_cast<const int32_t*>(cu_seqlens), N, T, HQ,
-                      HV, scale, h, h_chunks, d_out, d_final_state, dq, dk, dv, dg, dbeta,
-                      d_initial_state, ws, st);
-  return launch_bwd(q, k, v, A_log, a, dt_bias, b, static_cast<const int64_t*>(cu_seqlens), N, T, HQ, HV,
-                    scale, h, h_chunks, d_out, d_final_state, dq, dk, dv, dg, dbeta, d_initial_state, ws,
-                    st);
+  auto launch = [&](auto* cu) {
+    return launch_bwd(q, k, v, A_log, a, dt_bias, b, cu, N, T, HQ, HV, scale, h, h_chunks, d_out,
+                      d_final_state, dq, dk, dv, dg, dbeta, static_cast<float*>(nullptr),
+                      static_cast<float*>(nullptr), d_initial_state, ws, st);
+  };
+  return cu_is_int32 ? launch(static_cast<const int32_t*>(cu_seqlens))
+                     : launch(static_cast<const int64_t*>(cu_seqlens));
+}
+
+extern "C" int gdn_prefill_bwd_step(const uint16_t* q, const uint16_t* k, const uint16_t* v,
+                                    const float* A_log, const uint16_t* a, const float* dt_bias,
+                                    const uint16_t* b, const void* cu_seqlens, int cu_is_int32, int N,
+                                    int T, int HQ, int HV, float scale, const uint16_t* h, int h_chunks,
+                                    const uint16_t* d_out, const float* d_final_state, uint16_t* dq,
+                                    uint16_t* dk, uint16_t* dv, uint16_t* da, uint16_t* db, float* dA_log,
+                                    float* ddt_bias, float* d_initial_state, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  const int rc = check_bwd(q, k, v, A_log, a, dt_bias, b, cu_seqlens, N, T, HQ, HV, h, h_chunks, d_out,
+                           dq && dk && dv && da && db);
+  if (rc != GDN_OK) return rc;
+  if (!dA_log || !ddt_bias) return GDN_ERR_NULL;
+  if (workspace_bytes < gdn_prefill_bwd_workspace_bytes(N, T, HQ, HV) || (N > 0 && !workspace))
+    return GDN_ERR_WORKSPACE;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  auto launch = [&](auto* cu) {
+    return launch_bwd(q, k, v, A_log, a, dt_bias, b, cu, N, T, HQ, HV, scale, h, h_chunks, d_out,
+                      d_final_state, dq, dk, dv, da, db, dA_log, ddt_bias, d_initial_state, ws, st);
+  };
+  return cu_is_int32 ? launch(static_cast<const int32_t*>(cu_seqlens))
+                     : launch(static_cast<const int64_t*>(cu_seqlens));
 }
 
 extern "C" int gdn_gate_bwd(const float* A_log, const uint16_t* a, const float* dt_bias, const uint16_t* b,
