@@ -14,8 +14,8 @@
 //   Vn = Tm X, O = scale E Q S^T + P Vn, S' = e^{gam_L} S + Vn^T Dc K,
 // and its reverse is arranged in three launches:
 //
-//  1. gdn_bwd_prep_kernel, one workgroup per (chunk, v-head), all chunks at
-//     once: the state-gradient transition of the chunk,
+//  1. gdn_bwd_prep_kernel, persistent workgroups over the (chunk, v-head)
+//     units, all chunks at once: the state-gradient transition of the chunk,
 //        M = e^{gam_L} I - W2^T (beta E K),   W2 = Tm^T Dc K            [K x K]
 //        R = dO^T (scale E Q) - G1^T (beta E K),  G1 = Tm^T P^T dO      [V x K]
 //     so that dS = dSn M + R.  M is written as ready MFMA A-operand
@@ -64,11 +64,11 @@ namespace {
 
 using namespace gdn;
 
-constexpr int LDK = D + 8;           // [*][128] bf16 rows (272 B)
+// [*][128] bf16 LDS rows of 272 B: the packed 8-byte writes of 16 tokens then
+// hit distinct banks (288 B, which favours the 16-byte reads instead, made
+// the gradient kernel 1% slower).
+constexpr int LDK = D + 8;
 constexpr int LDC = C + 8;           // [*][64] bf16 rows (144 B)
-constexpr int LDA = C + 4;           // [64][64] fp32 rows (272 B)
-constexpr int kCB = C * LDK;         // elements of a [64][128] buffer
-constexpr int kTB = C * LDC;         // elements of a [64][64] buffer
 constexpr size_t kMBytes = size_t(D) * D * 2;   // M record (bf16 fragments)
 constexpr size_t kRBytes = size_t(D) * D * 2;   // R record (bf16, accumulator layout); then dSn (bf16 [v][k])
 constexpr size_t kTmBytes = size_t(C) * C * 2;  // Tm record (bf16 [t][t'], zero above the diagonal)
@@ -96,12 +96,39 @@ __device__ __forceinline__ bf16x8_t op_rm(const uint16_t* base, int ld, int m0, 
   return __builtin_bit_cast(bf16x8_t, v);
 }
 
-// Accumulator tile (lane l holds rows r0 + 4 (l / 16) + i, column c0 + l % 16)
-// to a bf16 matrix stored [row][col] / transposed [col][row].
-__device__ __forceinline__ void st_tile(uint16_t* base, int ld, int r0, int c0, const f32x4& x, int lane) {
-  uint16_t* p = base + (r0 + 4 * (lane >> 4)) * ld + c0 + (lane & 15);
+// op_rm with the reduction slots in the order of two stacked accumulator
+// tiles: slot e of lane group q is row r0 + 16 (e / 4) + 4 q + e % 4.
+__device__ __forceinline__ bf16x8_t op_rmp(const uint16_t* base, int ld, int m0, int r0, int lane) {
+  const int j = lane & 15;
+  const uint16_t* p = base + (r0 + 4 * (lane >> 4) + (j >> 2)) * ld + m0 + 4 * (j & 3);
+  const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)p);
+  const i16x4_t hi =
+      __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(p + 16 * ld));
+  const i16x8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// An operand's 8 values times f0 (slots 0-3) and f1 (slots 4-7), rounded back to bf16.
+__device__ __forceinline__ bf16x8_t scale_bf8(bf16x8_t x, const f32x4& f0, const f32x4& f1) {
+  f32x4 lo, hi;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) p[i * ld] = f32_to_bf16_bits(x[i]);
+  for (int e = 0; e < 4; ++e) {
+    lo[e] = f0[e] * float(x[e]);
+    hi[e] = f1[e] * float(x[4 + e]);
+  }
+  return pack2_bf(lo, hi);
+}
+
+// 4 adjacent bf16 values as floats, and back (round to nearest even).
+__device__ __forceinline__ f32x4 bf4_f32(const uint2& w) {
+  float x0, x1, x2, x3;
+  unpack_bf16x2(w.x, x0, x1);
+  unpack_bf16x2(w.y, x2, x3);
+  return f32x4{x0, x1, x2, x3};
+}
+
+__device__ __forceinline__ void st_bf4(uint16_t* p, const f32x4& x) {
+  *reinterpret_cast<uint2*>(p) = uint2{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3])};
 }
 
 // Sum over the 4 lane groups (same lane % 16) of a wave, in every lane: a
@@ -123,13 +150,14 @@ constexpr int GB_DA = GB_SZ, GB_DB = GB_SZ + C, GB_G = GB_SZ + 2 * C;   // GateF
 // The gate inputs of token `lane` of the chunk (wave 0): loaded early, used
 // by chunk_gates_calc once the chunk's rows are on their way.
 struct GateIn {
-  float a, b, dt, alog;
+  uint16_t a, b;       // as loaded: converted where they are used, so that nothing waits for them before
+  float dt, alog;
 };
 
 __device__ __forceinline__ GateIn gate_inputs(const float* A_log, const uint16_t* a, const float* dt_bias,
                                               const uint16_t* b, int HV, int hv, int t0, int len, int lane) {
   const size_t i = size_t(t0 + min(lane, len - 1)) * HV + hv;
-  return GateIn{bf16_bits_to_f32(a[i]), bf16_bits_to_f32(b[i]), dt_bias[hv], A_log[hv]};
+  return GateIn{a[i], b[i], dt_bias[hv], A_log[hv]};
 }
 
 // g = -exp(A_log) softplus(a + dt_bias), beta = sigmoid(b) per token (zero
@@ -139,10 +167,10 @@ __device__ __forceinline__ void chunk_gates_calc(const GateIn& in, int len, int 
   constexpr float kLog2e = 1.44269504088896341f, kLn2 = 0.69314718055994531f;
   float g = 0.f, be = 0.f;
   if (lane < len) {
-    const float x = in.a + in.dt;
+    const float x = bf16_bits_to_f32(in.a) + in.dt;
     const float sp = fmaxf(x, 0.f) + kLn2 * __builtin_amdgcn_logf(1.f + __builtin_amdgcn_exp2f(-fabsf(x) * kLog2e));
     g = -__builtin_amdgcn_exp2f(in.alog * kLog2e) * sp;
-    be = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-in.b * kLog2e));
+    be = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-bf16_bits_to_f32(in.b) * kLog2e));
   }
   const float gam = wave_inclusive_scan(g);
   const float gl = __shfl(gam, 63);
@@ -156,354 +184,432 @@ __device__ __forceinline__ void chunk_gates_calc(const GateIn& in, int len, int 
   }
 }
 
-// Rows [t0, t0 + len) of a [*, stride] bf16 tensor (128 columns) into a
-// [64][LDK] LDS buffer, rows past len zero, in two steps so that the HBM
-// reads of several tensors are in flight together: rows_fetch issues this
-// thread's 16-byte reads (2 of the 1024 of a tensor, 512 threads), rows_store
-// writes them.
-__device__ __forceinline__ void rows_fetch(uint4 (&w)[2], const uint16_t* src, size_t stride, int t0,
-                                           int len, int tid) {
+// One chunk's rows of one head of a [T, heads, 128] tensor, as a buffer from
+// token t0's row: byte offset (t * heads * 128 + column) * sizeof(T) of token
+// t0 + t.  Rows at or past len fall outside it (a load gives zeros, a store
+// writes nothing), so the accesses need no branch and every path through a
+// loop issues the same memory instructions: with branches around them the
+// compiler's waits for the next step's loads also waited for stores issued
+// after them.
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t head_rows(T* base, int heads, int head, int t0, int len) {
+  return uniform_buffer(base + (size_t(t0) * heads + head) * D,
+                        len > 0 ? uint32_t((len * heads - head) * D * int(sizeof(T))) : 0u);
+}
+
+__device__ __forceinline__ uint4 buffer_load_b128(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, int(off), 0, 0));
+}
+__device__ __forceinline__ uint2 buffer_load_b64(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, int(off), 0, 0));
+}
+
+// A chunk's 64 rows into a [64][LDK] LDS buffer, rows past the chunk zero, in
+// two steps so that the HBM reads of several tensors are in flight together:
+// rows_fetch issues this thread's 16-byte reads (of the 1024 of a tensor),
+// rows_store writes them.
+template <int kThreads>
+__device__ __forceinline__ void rows_fetch(uint4 (&w)[1024 / kThreads], __amdgpu_buffer_rsrc_t src, int heads,
+                                           int tid) {
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int x = tid + it * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
-    w[it] = r < len ? *reinterpret_cast<const uint4*>(src + size_t(t0 + r) * stride + cc)
-                    : make_uint4(0, 0, 0, 0);
+  for (int it = 0; it < 1024 / kThreads; ++it) {
+    const int x = tid + it * kThreads;
+    w[it] = buffer_load_b128(src, uint32_t((x >> 4) * heads * D + (x & 15) * 8) * 2u);
   }
 }
 
-__device__ __forceinline__ void rows_store(uint16_t* dst, const uint4 (&w)[2], int tid) {
+template <int kThreads>
+__device__ __forceinline__ void rows_store(uint16_t* dst, const uint4 (&w)[1024 / kThreads], int tid) {
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int x = tid + it * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
+  for (int it = 0; it < 1024 / kThreads; ++it) {
+    const int x = tid + it * kThreads, r = x >> 4, cc = (x & 15) * 8;
     *reinterpret_cast<uint4*>(dst + r * LDK + cc) = w[it];
-  }
-}
-
-// A 128 x 128 bf16 state (rows of 256 B in HBM) into a [128][LDK] LDS buffer,
-// in the same two steps (4 reads per thread).
-__device__ __forceinline__ void state_fetch(uint4 (&w)[4], const uint16_t* src, int tid) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) w[it] = reinterpret_cast<const uint4*>(src)[tid + it * kGradThreads];
-}
-
-__device__ __forceinline__ void state_store(uint16_t* dst, const uint4 (&w)[4], int tid) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int x = tid + it * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
-    *reinterpret_cast<uint4*>(dst + r * LDK + cc) = w[it];
-  }
-}
-
-// (I + A)^-1 of the strictly lower A = diag(beta) Ar (fp32 [64][LDA] in LDS,
-// zero on and above the diagonal), one wave, in fp32:
-//   * the four diagonal 16 x 16 blocks by forward substitution, lane l taking
-//     column l % 16 of block l / 16:  x_r = delta_rc - beta_r sum_{m<r} Ar_rm x_m;
-//   * the blocks below them block-row by block-row,
-//     T_ij = -T_ii (sum_{j<=m<i} A_im T_mj), on fp32 MFMA 16x16x4, each
-//     product's sum staged through sZ (16 x 17 floats).
-// The fp32 blocks go to sT ([64][LDA]), the bf16 result (zero above the
-// diagonal) to sTm [i][j].  The wave's LDS operations complete in order, so
-// its own writes are visible to its later reads without a barrier.
-__device__ __forceinline__ void unit_lower_inverse(const float* sAr, const float* gb, float* sT,
-                                                   float* sZ, uint16_t* sTm, int lane) {
-  const int bi = lane >> 4, c = lane & 15;
-  {
-    float x[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) x[r] = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 16 * bi + r;
-      float acc = 0.f;
-#pragma unroll
-      for (int m = 0; m < r; m += 4) {
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(&sAr[row * LDA + 16 * bi + m]);
-        acc = fmaf(a4[0], x[m], acc);
-        acc = fmaf(a4[1], x[m + 1], acc);
-        acc = fmaf(a4[2], x[m + 2], acc);
-        acc = fmaf(a4[3], x[m + 3], acc);
-      }
-      x[r] = (r == c ? 1.f : 0.f) - gb[GB_BETA + row] * acc;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 16 * bi + r;
-      sT[row * LDA + 16 * bi + c] = x[r];
-#pragma unroll
-      for (int jb = 0; jb < 4; ++jb)
-        if (jb != bi) sTm[row * LDC + 16 * jb + c] = 0;
-      sTm[row * LDC + 16 * bi + c] = f32_to_bf16_bits(x[r]);
-    }
-  }
-  const int q = lane >> 4;
-#pragma unroll
-  for (int i = 1; i < 4; ++i) {
-#pragma unroll
-    for (int j = i - 1; j >= 0; --j) {
-      f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      const float be = gb[GB_BETA + 16 * i + c];
-#pragma unroll
-      for (int m = j; m < i; ++m)
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const float a = be * sAr[(16 * i + c) * LDA + 16 * m + 4 * s4 + q];
-          const float b = sT[(16 * m + 4 * s4 + q) * LDA + 16 * j + c];
-          z = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, z, 0, 0, 0);
-        }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sZ[(4 * q + e) * 17 + c] = z[e];
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const float a = sT[(16 * i + c) * LDA + 16 * i + 4 * s4 + q];
-        const float b = sZ[(4 * s4 + q) * 17 + c];
-        t = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, t, 0, 0, 0);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = 16 * i + 4 * q + e;
-        sT[row * LDA + 16 * j + c] = -t[e];
-        sTm[row * LDC + 16 * j + c] = f32_to_bf16_bits(-t[e]);
-      }
-    }
-  }
-}
-
-// Decayed, masked K K^T (strict: Ar, fp32) or scaled Q K^T (inclusive: P,
-// bf16) tile (ti, tj) of the chunk from K / Q rows in LDS.
-template <bool kP>
-__device__ __forceinline__ void kk_tile(const uint16_t* sX, const uint16_t* sK, const float* gb, int ti,
-                                        int tj, float scale, float* sAr, uint16_t* sP, int lane) {
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < D / 32; ++s)
-    acc = mfma16_bf(op_mr(sX, LDK, 16 * ti, 32 * s, lane), op_mr(sK, LDK, 16 * tj, 32 * s, lane), acc);
-  const int col = 16 * tj + (lane & 15);
-  const float gc = gb[GB_GAM + col];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 16 * ti + 4 * (lane >> 4) + i;
-    const bool keep = kP ? row >= col : row > col;
-    const float v = keep ? acc[i] * expf(gb[GB_GAM + row] - gc) : 0.f;
-    if constexpr (kP) sP[row * LDC + col] = f32_to_bf16_bits(scale * v);
-    else sAr[row * LDA + col] = v;
-  }
-}
-
-// The 20 tiles of Ar and P on or below the diagonal, spread over 8 waves.
-__device__ __forceinline__ void ar_p_tiles(const uint16_t* sK, const uint16_t* sQ, const float* gb,
-                                           float scale, float* sAr, uint16_t* sP, int wave, int lane) {
-  for (int job = wave; job < 20; job += 8) {
-    const int t = job % 10;
-    const int ti = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
-    const int tj = t - (ti * (ti + 1)) / 2;
-    if (job < 10) kk_tile<false>(sK, sK, gb, ti, tj, scale, sAr, sP, lane);
-    else kk_tile<true>(sQ, sK, gb, ti, tj, scale, sAr, sP, lane);
   }
 }
 
 // ---------------------------------------------------------------------------
-// 1. Transition of the state gradient per (chunk, v-head): M and R.
+// 1. Transition of the state gradient per (chunk, v-head): M, R and Tm.
 //
 // M record: 32 fragments of 1 KB, fragment (kt, s) = kt * 4 + s holds for
 // lane l the 8 bf16 of M^T[16 kt + l % 16][j] at j = 32 s + 16 (e / 4) +
 // 4 (l / 16) + e % 4, e = 0..7: the A operand of the chain kernel's product
 // dS^T M-side, whose B operand is two stacked accumulator tiles of dS^T.
-// R record: R^T tiles (kt, vt), vt-major, lane l's 4 values (bf16, 8 bytes)
-// at 8 l: rows 16 kt + 4 (l / 16) + i, column 16 vt + l % 16 -- the chain
-// kernel's accumulator layout.  bf16 like M and like the dSn operand the
-// chain multiplies by M: R enters dS = dSn M + R with the same rounding.
+// R record: R^T tiles in pairs (kt, kt + 1) of a row block vt, vt-major,
+// lane l's 2 x 4 values (bf16, 16 bytes) at 16 l: rows 16 kt + 4 (l / 16) + i,
+// column 16 vt + l % 16 -- the chain kernel's accumulator layout.  bf16 like
+// M and like the dSn operand the chain multiplies by M: R enters dS = dSn M +
+// R with the same rounding.
+//
+// Bound by HBM at 32 768 tokens qk16/v32: 0.36 ms for the 2.0 GB it must move
+// (5.6 TB/s).  It replaces a form that took 0.97 ms: one workgroup of 8 waves
+// per CU (160 KB of LDS, scaled copies of K and Q among it) whose other waves
+// waited for one wave's inverse of the whole block.
+// Workgroups of 4 waves, two per CU (78 KB of LDS each), so that one's serial
+// inverse overlaps the other's products and stores:
+//   P1  the lower 16x16 tiles of A (fp32) and P; wave w inverts A's diagonal
+//       tile w by forward substitution
+//   P2  wave j: the blocks below the diagonal of block column j of
+//       Tm = (I + A)^-1, T_ij = -T_ii sum_m A_im T_mj, on fp32 MFMA (a block
+//       column needs no other); every wave: G0 = P^T dO for its 32 columns
+//   P3  W2, G1, M and R for the wave's 32 columns, operands from the wave's
+//       own accumulators and transposing reads of K and Q as loaded: the row
+//       factors beta E, scale E and Dc are applied to the other operand, in
+//       fp32 where that is an accumulator
+// All reductions over tokens take them in the order of stacked accumulator
+// tiles (op_rmp).
+constexpr int kPrepThreads = 256;
+
+// Forward substitution of one unit lower triangular 16 x 16 block I + A
+// (A fp32 [16][16] in LDS, strictly lower), lane l taking column l % 16:
+// x_r = delta_rc - sum_{m<r} A_rm x_m, column by column.
+__device__ __forceinline__ void unit_lower_inverse16(const float* sA, int c, float (&x)[16]) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x[r] = r == c ? 1.f : 0.f;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    f32x4 a[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (r > 4 * mb) a[r] = *reinterpret_cast<const f32x4*>(sA + 16 * r + 4 * mb);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (r > 4 * mb + e) x[r] = fmaf(-a[r][e], x[4 * mb + e], x[r]);
+  }
+}
+
 template <typename CuT>
-__global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_prep_kernel(
+__global__ __launch_bounds__(kPrepThreads, 2) void gdn_bwd_prep_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const float* __restrict__ A_log,
     const uint16_t* __restrict__ a, const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
     const CuT* __restrict__ cu, int N, int T, int HQ, int HV, float scale,
-    const uint16_t* __restrict__ d_out, int h_chunks, int slots, char* __restrict__ mrec,
+    const uint16_t* __restrict__ d_out, int h_chunks, int slots, int heads, char* __restrict__ mrec,
     char* __restrict__ rrec, uint16_t* __restrict__ tmrec, int2* __restrict__ chunks) {
-  __shared__ __align__(16) uint16_t sK[kCB];      // K; then G0 = P^T dO
-  __shared__ __align__(16) uint16_t sQ[kCB];      // Q; then W2 = Tm^T Dc K
-  __shared__ __align__(16) uint16_t sdO[kCB];
-  __shared__ __align__(16) uint16_t sDK[kCB];     // Dc K
-  __shared__ __align__(16) uint16_t sBEK[kCB];    // beta E K
-  __shared__ __align__(16) uint16_t sEQ[kCB];     // scale E Q
-  __shared__ __align__(16) float sAr[C * LDA];    // Ar; then -G1 (bf16 [64][LDK])
-  __shared__ __align__(16) uint16_t sP[kTB];
-  __shared__ __align__(16) uint16_t sTm[kTB];
-  __shared__ __align__(16) float sT[C * LDA];     // fp32 Tm blocks (the inverse's own)
-  __shared__ __align__(16) float sZ[16 * 17];
-  __shared__ __align__(16) float gb[GB_SZ];
+  __shared__ __align__(16) uint16_t sK[C * LDK];
+  __shared__ __align__(16) uint16_t sQ[C * LDK];
+  __shared__ __align__(16) uint16_t sdO[C * LDK];     // dO; then Tm ([64][LDC])
+  __shared__ __align__(16) uint16_t sP[C * LDC];
+  __shared__ __align__(16) float sA[10][16 * 16];     // lower tiles of A, row by row
+  __shared__ __align__(16) float sD[4][16 * 16];      // the inverses of the diagonal tiles
+  __shared__ __align__(16) float gbuf[2][GB_SZ];
+  __shared__ int4 next_unit[2];
+  uint16_t* sTm = sdO;
 
   const int tid0 = threadIdx.x, lane0 = tid0 & 63;
-  const int tid = tid0, lane = lane0;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Persistent workgroups (one per CU: the LDS holds one): workgroup w takes
-  // the (chunk slot, v-head) units w, w + gridDim.x, ... (slot fastest, the
-  // order of a (slots, HV) grid) and fetches the next unit's rows and gate
-  // inputs into registers while it works on one, so the HBM latency of a
-  // unit's inputs is spent inside the unit before it.
-  const int units = slots * HV;
-  auto locate = [&](int u, int& t0, int& len) {
-    const int slot = u % slots;
-    if (slot >= h_chunks) return false;
-    int n, ci;
-    locate_chunk(cu, N, T, slot, lane, n, ci);
-    if (n < 0) return false;
-    int bos, slen;
-    seq_bounds(cu, n, T, bos, slen);
-    t0 = bos + C * ci;
-    len = min(C, slen - C * ci);
-    return true;
+  const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+  // Persistent workgroups walk the units -- a chunk slot and `heads` v-heads
+  // of one qk-head, v-heads fastest -- and a unit's v-heads in turn.  The next
+  // step's rows and gate inputs are loaded into registers while this one is
+  // worked on; wave 3 looks up the unit after the next.
+  const int groups = HV / heads, units = slots * groups;
+  struct At {
+    int unit, m, t0, len;
   };
-  auto fetch = [&](int u, int t0, int len, uint4 (&wk)[2], uint4 (&wq)[2], uint4 (&wo)[2], GateIn& gi) {
-    const int hv = u / slots, hq = hv / (HV / HQ);
-    if (wave == 0) gi = gate_inputs(A_log, a, dt_bias, b, HV, hv, t0, len, lane);
-    rows_fetch(wk, k + size_t(hq) * D, size_t(HQ) * D, t0, len, tid);
-    rows_fetch(wq, q + size_t(hq) * D, size_t(HQ) * D, t0, len, tid);
-    rows_fetch(wo, d_out + size_t(hv) * D, size_t(HV) * D, t0, len, tid);
-  };
-  uint4 wk[2], wq[2], wo[2];
-  GateIn gi{};
-  int t0 = 0, len = 0;
-  bool ok = int(blockIdx.x) < units && locate(int(blockIdx.x), t0, len);
-  if (ok) fetch(int(blockIdx.x), t0, len, wk, wq, wo, gi);
-  for (int u = int(blockIdx.x); u < units; u += int(gridDim.x)) {
-    // the slot's token range for the gradient kernel (length 0: no chunk)
-    if (u < slots && tid0 == 0) chunks[u] = int2{t0, ok ? len : 0};
-    // the next unit's inputs, in flight while this one is worked on
-    const int un = u + int(gridDim.x);
-    int t0n = 0, lenn = 0;
-    const bool okn = un < units && locate(un, t0n, lenn);
-    uint4 wkn[2], wqn[2], won[2];
-    GateIn gin{};
-    if (okn) fetch(un, t0n, lenn, wkn, wqn, won, gin);
-    if (ok) {
-      const int slot = u % slots, hv = u / slots;
-      // Lane indices opaque to the compiler at the top of each unit: their
-      // address arithmetic is formed where it is used instead of being
-      // hoisted out of the loop into registers live across every unit.
-      int tid = tid0, lane = lane0;
-      asm volatile("" : "+v"(tid), "+v"(lane));
-      for (int x = tid; x < C * LDA; x += kGradThreads) sAr[x] = 0.f;
-      for (int x = tid; x < kTB; x += kGradThreads) sP[x] = 0;
-      rows_store(sK, wk, tid);
-      rows_store(sQ, wq, tid);
-      rows_store(sdO, wo, tid);
-      if (wave == 0) chunk_gates_calc(gi, len, lane, gb);
-      lds_barrier();
-
-      // Ar, P; the scaled row copies
-      ar_p_tiles(sK, sQ, gb, scale, sAr, sP, wave, lane);
-      for (int x = tid; x < C * 16; x += kGradThreads) {
-        const int r = x >> 4, cc = (x & 15) * 8;
-        const uint4 kw = *reinterpret_cast<const uint4*>(&sK[r * LDK + cc]);
-        const uint4 qw = *reinterpret_cast<const uint4*>(&sQ[r * LDK + cc]);
-        const float fd = gb[GB_DC + r], fb = gb[GB_BETA + r] * gb[GB_E + r], fq = scale * gb[GB_E + r];
-        const uint32_t kk[4] = {kw.x, kw.y, kw.z, kw.w}, qq[4] = {qw.x, qw.y, qw.z, qw.w};
-        uint32_t od[4], ob[4], oq[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float k0, k1, q0, q1;
-          unpack_bf16x2(kk[e], k0, k1);
-          unpack_bf16x2(qq[e], q0, q1);
-          od[e] = pack_bf16x2(fd * k0, fd * k1);
-          ob[e] = pack_bf16x2(fb * k0, fb * k1);
-          oq[e] = pack_bf16x2(fq * q0, fq * q1);
-        }
-        *reinterpret_cast<uint4*>(&sDK[r * LDK + cc]) = make_uint4(od[0], od[1], od[2], od[3]);
-        *reinterpret_cast<uint4*>(&sBEK[r * LDK + cc]) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
-        *reinterpret_cast<uint4*>(&sEQ[r * LDK + cc]) = make_uint4(oq[0], oq[1], oq[2], oq[3]);
-      }
-      lds_barrier();
-
-      // Tm (wave 0) while waves 1-7 form G0 = P^T dO [t][v] over sK (K is done)
-      if (wave == 0) {
-        unit_lower_inverse(sAr, gb, sT, sZ, sTm, lane);
-      } else {
-        for (int x = wave - 1; x < 32; x += 7) {
-          const int tb = x & 3, vb = x >> 2;
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int s = 0; s < C / 32; ++s)
-            acc = mfma16_bf(op_rm(sP, LDC, 16 * tb, 32 * s, lane), op_rm(sdO, LDK, 16 * vb, 32 * s, lane), acc);
-          st_tile(sK, LDK, 16 * tb, 16 * vb, acc, lane);
+  // the first unit at or after `unit` (in this workgroup's stride) that holds
+  // a chunk (unit >= units: none); wave 3 notes the token range of every slot
+  // it passes for the gradient kernel (length 0: no chunk)
+  auto seek = [&](int unit) {
+    At x{unit, 0, 0, 0};
+    for (; x.unit < units; x.unit += int(gridDim.x)) {
+      const int slot = x.unit / groups;
+      x.len = 0;
+      if (slot < h_chunks) {
+        int n, ci;
+        locate_chunk(cu, N, T, slot, lane0, n, ci);
+        if (n >= 0) {
+          int bos, slen;
+          seq_bounds(cu, n, T, bos, slen);
+          x.t0 = __builtin_amdgcn_readfirstlane(bos + C * ci);
+          x.len = __builtin_amdgcn_readfirstlane(min(C, slen - C * ci));
         }
       }
-      lds_barrier();
+      if (wave == 3 && lane0 == 0 && x.unit == slot * groups) chunks[slot] = int2{x.t0, x.len};
+      if (x.len > 0) break;
+    }
+    return x;
+  };
+  auto head_of = [&](const At& x) { return (x.unit % groups) * heads + x.m; };
+  struct Regs {
+    uint4 k[4], q[4], o[4];
+  };
+  auto fetch = [&](const At& x, Regs& r, int tid) {
+    const int hv = head_of(x), hq = hv / (HV / HQ);
+    if (x.m == 0) {
+      rows_fetch<kPrepThreads>(r.k, head_rows(k, HQ, hq, x.t0, x.len), HQ, tid);
+      rows_fetch<kPrepThreads>(r.q, head_rows(q, HQ, hq, x.t0, x.len), HQ, tid);
+    }
+    rows_fetch<kPrepThreads>(r.o, head_rows(d_out, HV, hv, x.t0, x.len), HV, tid);
+  };
+  auto gate_in = [&](const At& x, int lane) {
+    return gate_inputs(A_log, a, dt_bias, b, HV, head_of(x), x.t0, x.len, lane);
+  };
 
-      // Tm for the gradient kernel
-      reinterpret_cast<uint4*>(tmrec + (size_t(slot) * HV + hv) * C * C)[tid] =
-          *reinterpret_cast<const uint4*>(sTm + (tid >> 3) * LDC + 8 * (tid & 7));
-      // W2 = Tm^T Dc K -> sQ, -G1 = -Tm^T G0 -> sAr (as bf16 [64][LDK])
-      uint16_t* sG1 = reinterpret_cast<uint16_t*>(sAr);
-      {
-        const int tb = wave & 3, d0 = 4 * (wave >> 2);
+  // the tiles of sP above the diagonal that an operand read covers stay zero
+  for (int x = tid0; x < 2 * 16 * 16; x += kPrepThreads) {
+    const int up = x >> 8, r = (x >> 4) & 15, c = x & 15;
+    sP[(32 * up + r) * LDC + 32 * up + 16 + c] = 0;
+  }
+
+  At at = seek(int(blockIdx.x));
+  if (at.unit >= units) return;
+  At after = seek(at.unit + int(gridDim.x));      // the unit after at's
+  Regs cur;
+  fetch(at, cur, tid0);
+  if (wave == 3) chunk_gates_calc(gate_in(at, lane0), at.len, lane0, gbuf[0]);
+  // This wave's tiles (ti, tj) of A and P: diagonal tile `wave` and one or two
+  // below the diagonal; their Q K^T and K K^T, transposed (rows s = 16 tj +
+  // 4 g + i, column t = 16 ti + c), serve all v-heads of the unit.
+  const int ti1 = wave == 0 ? 1 : wave == 3 ? 3 : 2, tj1 = wave < 2 ? 0 : 1;
+  const int ti2 = 3, tj2 = wave == 2 ? 0 : 2;
+  const bool three = wave >= 2;
+  f32x4 qk[3], kk[3];
+  for (int it = 0, un = 0; at.unit < units; ++it) {
+    // Lane indices opaque to the compiler at the top of each phase: their
+    // address arithmetic is formed where it is used instead of being kept in
+    // registers across phases and steps.
+    int tid = tid0, lane = lane0, g, c;
+    auto fresh_lane = [&] {
+      asm volatile("" : "+v"(lane), "+v"(tid));
+      g = lane >> 4;
+      c = lane & 15;
+    };
+    fresh_lane();
+    const int slot = at.unit / groups, hv = head_of(at), m = at.m;
+    const float* gb = gbuf[it & 1];
+    const size_t rec = size_t(slot) * HV + hv;
+    if (m == 0) {
+      rows_store<kPrepThreads>(sK, cur.k, tid);
+      rows_store<kPrepThreads>(sQ, cur.q, tid);
+    }
+    rows_store<kPrepThreads>(sdO, cur.o, tid);
+    lds_barrier();
+
+    // P1: the tiles; dO as operands of this wave's columns v = 32 wave + 16 u + c
+    bf16x8_t dof[2][2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int db = d0 + u;
-          f32x4 w2 = {0.f, 0.f, 0.f, 0.f}, g1 = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 2; ++s)
 #pragma unroll
-          for (int s = 0; s < C / 32; ++s) {
-            const bf16x8_t tmt = op_rm(sTm, LDC, 16 * tb, 32 * s, lane);
-            w2 = mfma16_bf(tmt, op_rm(sDK, LDK, 16 * db, 32 * s, lane), w2);
-            g1 = mfma16_bf(tmt, op_rm(sK, LDK, 16 * db, 32 * s, lane), g1);
+      for (int u = 0; u < 2; ++u) dof[s][u] = op_rmp(sdO, LDK, 32 * wave + 16 * u, 32 * s, lane);
+    auto tiles = [&](auto count) {
+#pragma unroll
+      for (int j = 0; j < decltype(count)::value; ++j) {
+        const int ti = j == 0 ? wave : j == 1 ? ti1 : ti2, tj = j == 0 ? wave : j == 1 ? tj1 : tj2;
+        if (m == 0) {
+          f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const bf16x8_t ka = op_mr(sK, LDK, 16 * tj, 32 * s, lane);
+            x = mfma16_bf(ka, op_mr(sQ, LDK, 16 * ti, 32 * s, lane), x);
+            y = mfma16_bf(ka, op_mr(sK, LDK, 16 * ti, 32 * s, lane), y);
           }
-          st_tile(sQ, LDK, 16 * tb, 16 * db, w2, lane);
-          st_tile(sG1, LDK, 16 * tb, 16 * db, -g1, lane);
+          qk[j] = x;
+          kk[j] = y;
+        }
+        const int t = 16 * ti + c, s0 = 16 * tj + 4 * g;
+        const float gt = gb[GB_GAM + t], be = gb[GB_BETA + t];
+        const f32x4 gs = *reinterpret_cast<const f32x4*>(&gb[GB_GAM + s0]);
+        f32x4 pv, av;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float ex = t >= s0 + i ? exp_fast(gt - gs[i]) : 0.f;
+          pv[i] = scale * (ex * qk[j][i]);
+          av[i] = t > s0 + i ? be * (ex * kk[j][i]) : 0.f;
+        }
+        st_bf4(sP + t * LDC + s0, pv);
+        *reinterpret_cast<f32x4*>(&sA[(ti * (ti + 1)) / 2 + tj][16 * c + 4 * g]) = av;
+      }
+    };
+    if (three) tiles(IC<3>());
+    else tiles(IC<2>());
+    {
+      // a wave's LDS operations complete in order: its own tile needs no barrier
+      float x[16];
+      unit_lower_inverse16(sA[(wave * (wave + 1)) / 2 + wave], c, x);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        sD[wave][16 * (4 * g + i) + c] = g == 0 ? x[i] : g == 1 ? x[4 + i] : g == 2 ? x[8 + i] : x[12 + i];
+    }
+    At nx = at;
+    ++nx.m;
+    if (nx.m == heads) nx = after;
+    const bool more = nx.unit < units;
+    GateIn gin{};
+    if (wave == 3 && more) gin = gate_in(nx, lane);
+    lds_barrier();
+
+    // P2: Tm; G0 = P^T dO
+    fresh_lane();
+    Regs nxt;
+    fetch(more ? nx : at, nxt, tid);
+    bf16x8_t g0[2][2];
+    {
+      f32x4 acc[4][2];
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) {
+        acc[tb][0] = acc[tb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = tb / 2; s < 2; ++s) {
+          const bf16x8_t po = op_rmp(sP, LDC, 16 * tb, 32 * s, lane);
+#pragma unroll
+          for (int u = 0; u < 2; ++u) acc[tb][u] = mfma16_bf(po, dof[s][u], acc[tb][u]);
         }
       }
-      lds_barrier();
-
-      // M = e^{gam_L} I - W2^T (beta E K): tiles (jt, kt); R^T = (scale E Q)^T dO + (beta E K)^T (-G1)
-      const size_t rec = size_t(slot) * HV + hv;
-      char* mr = mrec + rec * kMBytes;
-      char* rr = rrec + rec * kRBytes;
-      const float eL = gb[GB_EL];
-      {
-        const int jt = wave;
-#pragma unroll 2
-        for (int kt = 0; kt < 8; ++kt) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int s = 0; s < C / 32; ++s)
-            acc = mfma16_bf(op_rm(sQ, LDK, 16 * jt, 32 * s, lane), op_rm(sBEK, LDK, 16 * kt, 32 * s, lane), acc);
-          const int kcol = 16 * kt + (lane & 15);
-          float m[4];
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) g0[s][u] = pack2_bf(acc[2 * s][u], acc[2 * s + 1][u]);
+    }
+    auto st_tm = [&](int ti, int tj, const f32x4& x) {
+      uint16_t* p = sTm + (16 * ti + 4 * g) * LDC + 16 * tj + c;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i * LDC] = f32_to_bf16_bits(x[i]);
+    };
+    auto column = [&](auto col) {
+      constexpr int j = decltype(col)::value;
+      f32x4 x[4 - j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[0][e] = sD[j][16 * (4 * g + e) + c];
+      st_tm(j, j, x[0]);
+#pragma unroll
+      for (int i = j + 1; i < 4; ++i) {
+        f32x4 z = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int mm = j; mm < i; ++mm) {
+          const f32x4 av = *reinterpret_cast<const f32x4*>(&sA[(i * (i + 1)) / 2 + mm][16 * c + 4 * g]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) z = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], x[mm - j][e], z, 0, 0, 0);
+        }
+        const f32x4 dv = *reinterpret_cast<const f32x4*>(&sD[i][16 * c + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[e], z[e], y, 0, 0, 0);
+        x[i - j] = -y;
+        st_tm(i, j, x[i - j]);
+      }
+    };
+    if (wave == 0) column(IC<0>());
+    else if (wave == 1) column(IC<1>());
+    else if (wave == 2) column(IC<2>());
+    else {
+      column(IC<3>());
+#pragma unroll
+      for (int x = 0; x < 6; ++x) {           // zero above the diagonal
+        const int ti = x < 3 ? 0 : x < 5 ? 1 : 2, tj = x < 3 ? x + 1 : x < 5 ? x - 1 : 3;
+        *reinterpret_cast<uint2*>(sTm + (16 * ti + c) * LDC + 16 * tj + 4 * g) = uint2{0, 0};
+      }
+      if (more) chunk_gates_calc(gin, nx.len, lane, gbuf[(it + 1) & 1]);
+      if (m == 0 && after.unit < units) {
+        const At x = seek(after.unit + int(gridDim.x));
+        if (lane == 0) next_unit[un & 1] = int4{x.unit, x.t0, x.len, 0};
+      }
+    }
+    lds_barrier();
+
+    // P3
+    fresh_lane();
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const int y = tid + x * kPrepThreads;
+      reinterpret_cast<uint4*>(tmrec + rec * C * C)[y] =
+          *reinterpret_cast<const uint4*>(sTm + (y >> 3) * LDC + 8 * (y & 7));
+    }
+    bf16x8_t w2[2][2], g1[2][2];
+    {
+      // W2 = Tm^T Dc K and G1 = Tm^T G0, then times -beta E
+      f32x4 wa[4][2], ga[4][2];
+      bf16x8_t dk[2][2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const f32x4 d0 = *reinterpret_cast<const f32x4*>(&gb[GB_DC + 32 * s + 4 * g]);
+        const f32x4 d1 = *reinterpret_cast<const f32x4*>(&gb[GB_DC + 32 * s + 16 + 4 * g]);
+        const f32x4 e0 = *reinterpret_cast<const f32x4*>(&gb[GB_E + 32 * s + 4 * g]);
+        const f32x4 e1 = *reinterpret_cast<const f32x4*>(&gb[GB_E + 32 * s + 16 + 4 * g]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          dk[s][u] = scale_bf8(op_rmp(sK, LDK, 32 * wave + 16 * u, 32 * s, lane), d0, d1);
+          dof[s][u] = scale_bf8(dof[s][u], scale * e0, scale * e1);
+        }
+      }
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) wa[tb][u] = ga[tb][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = tb / 2; s < 2; ++s) {
+          const bf16x8_t tm = op_rmp(sTm, LDC, 16 * tb, 32 * s, lane);
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            wa[tb][u] = mfma16_bf(tm, dk[s][u], wa[tb][u]);
+            ga[tb][u] = mfma16_bf(tm, g0[s][u], ga[tb][u]);
+          }
+        }
+        const f32x4 be = *reinterpret_cast<const f32x4*>(&gb[GB_BETA + 16 * tb + 4 * g]);
+        const f32x4 e = *reinterpret_cast<const f32x4*>(&gb[GB_E + 16 * tb + 4 * g]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int jrow = 16 * jt + 4 * (lane >> 4) + i;
-            m[i] = (jrow == kcol ? eL : 0.f) - acc[i];
+            wa[tb][u][i] *= -be[i] * e[i];
+            ga[tb][u][i] *= -be[i] * e[i];
           }
-          uint2 w;
-          w.x = pack_bf16x2(m[0], m[1]);
-          w.y = pack_bf16x2(m[2], m[3]);
-          *reinterpret_cast<uint2*>(mr + ((kt * 4 + (jt >> 1)) * 64 + lane) * 16 + 8 * (jt & 1)) = w;
-        }
-        const int kt = wave;
-#pragma unroll 2
-        for (int vt = 0; vt < 8; ++vt) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int s = 0; s < C / 32; ++s) {
-            acc = mfma16_bf(op_rm(sEQ, LDK, 16 * kt, 32 * s, lane), op_rm(sdO, LDK, 16 * vt, 32 * s, lane), acc);
-            acc = mfma16_bf(op_rm(sBEK, LDK, 16 * kt, 32 * s, lane), op_rm(sG1, LDK, 16 * vt, 32 * s, lane), acc);
-          }
-          *reinterpret_cast<uint2*>(rr + ((vt * 8 + kt) * 64 + lane) * 8) =
-              uint2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
-        }
       }
-      // the next unit overwrites every buffer this one reads last
-      lds_barrier();
-    }
-    ok = okn;
-    t0 = t0n;
-    len = lenn;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      wk[i] = wkn[i];
-      wq[i] = wqn[i];
-      wo[i] = won[i];
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          w2[s][u] = pack2_bf(wa[2 * s][u], wa[2 * s + 1][u]);
+          g1[s][u] = pack2_bf(ga[2 * s][u], ga[2 * s + 1][u]);
+        }
     }
-    gi = gin;
+    // M = e^{gam_L} I - W2^T beta E K: rows j = 32 wave + 16 u + 4 g + i, column 16 kt + c.
+    // R^T = K^T (-beta E G1) + Q^T (scale E dO): rows 16 kt + 4 g + i, column v.
+    const float eL = gb[GB_EL];
+    char* mr = mrec + rec * kMBytes + wave * 1024 + lane * 16;
+    char* rr = rrec + rec * kRBytes + (8 * wave) * 1024 + lane * 16;
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp) {
+      uint2 rw[2][2];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        const int kt = 2 * kp + o;
+        bf16x8_t kf[2], qf[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          kf[s] = op_rmp(sK, LDK, 16 * kt, 32 * s, lane);
+          qf[s] = op_rmp(sQ, LDK, 16 * kt, 32 * s, lane);
+        }
+        uint2 mw[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f32x4 ma, ra = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ma[i] = kp == wave && o == u && 4 * g + i == c ? eL : 0.f;
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            ma = mfma16_bf(w2[s][u], kf[s], ma);
+            ra = mfma16_bf(kf[s], g1[s][u], ra);
+            ra = mfma16_bf(qf[s], dof[s][u], ra);
+          }
+          mw[u] = uint2{cvt_pk_bf16(ma[0], ma[1]), cvt_pk_bf16(ma[2], ma[3])};
+          rw[u][o] = uint2{cvt_pk_bf16(ra[0], ra[1]), cvt_pk_bf16(ra[2], ra[3])};
+        }
+        *reinterpret_cast<uint4*>(mr + kt * 4096) = uint4{mw[0].x, mw[0].y, mw[1].x, mw[1].y};
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        *reinterpret_cast<uint4*>(rr + (4 * u + kp) * 1024) =
+            uint4{rw[u][0].x, rw[u][0].y, rw[u][1].x, rw[u][1].y};
+    }
+    if (more && nx.m == 0) {
+      const int4 x = next_unit[un & 1];
+      after = At{__builtin_amdgcn_readfirstlane(x.x), 0, __builtin_amdgcn_readfirstlane(x.y),
+                 __builtin_amdgcn_readfirstlane(x.z)};
+      ++un;
+    }
+    // the next step overwrites what this one reads last
+    lds_barrier();
+    cur = nxt;
+    at = nx;
   }
 }
 
@@ -561,15 +667,15 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     for (int x = 0; x < kMCopies; ++x)
       lds_dma16_saddr(ms, uint32_t((x * kThreads + tid) * 16), &sM[buf][(x * kThreads + wave * 64) * 8]);
   };
-  auto fetch_r = [&](int ch, uint2 (&r)[8]) {
+  auto fetch_r = [&](int ch, uint4 (&r)[4]) {
     const char* rs = rrec + rec_of(ch) * kRBytes;
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt)
-      r[kt] = *reinterpret_cast<const uint2*>(rs + ((vb * 8 + kt) * 64 + lane) * 8);
+    for (int kp = 0; kp < 4; ++kp)
+      r[kp] = *reinterpret_cast<const uint4*>(rs + ((vb * 4 + kp) * 64 + lane) * 16);
   };
   // one chunk: dSn out, dS = dSn M + R (cur = R of chunk ch), and the copies
   // for chunk ch - 2 (R into nxt2, M into LDS buffer (it + 2) % 3)
-  auto step = [&](int ch, int it, uint2 (&cur)[8], uint2 (&nxt2)[8]) {
+  auto step = [&](int ch, int it, uint4 (&cur)[4], uint4 (&nxt2)[4]) {
     const int buf = it % 3;
     if (ch > 1) {
       copy_m(ch - 2, (it + 2) % 3);
@@ -588,8 +694,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     for (int s = 0; s < 4; ++s) bop[s] = pack2_bf(acc[2 * s], acc[2 * s + 1]);
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
-      acc[kt] = f32x4{__uint_as_float(cur[kt].x << 16), __uint_as_float(cur[kt].x & 0xffff0000u),
-                      __uint_as_float(cur[kt].y << 16), __uint_as_float(cur[kt].y & 0xffff0000u)};
+      acc[kt] = bf4_f32((kt & 1) ? uint2{cur[kt / 2].z, cur[kt / 2].w} : uint2{cur[kt / 2].x, cur[kt / 2].y});
 #pragma unroll
       for (int s = 0; s < 4; ++s)
         acc[kt] = mfma16_bf(ld16_bf(&sM[buf][((kt * 4 + s) * 64 + lane) * 8]), bop[s], acc[kt]);
@@ -597,11 +702,11 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     // Vector memory operations complete in issue order: with at most this
     // chunk's copies (M and R two chunks ahead) and its 8 dSn stores still
     // outstanding, everything the next chunk reads has landed.
-    if (ch > 1) wait_vm<kMCopies + 8 + 8>();
+    if (ch > 1) wait_vm<kMCopies + 4 + 8>();
     else wait_vm<8>();
     lds_barrier();
   };
-  uint2 r0[8], r1[8], r2[8];
+  uint4 r0[4], r1[4], r2[4];
   if (last >= 0) {
     copy_m(last, 0);
     fetch_r(last, r0);
@@ -691,18 +796,6 @@ struct GradParts {
   float vks[8];      // sum of Dc rowsum(Vn K dSn^T) per wave
 };
 
-// 4 adjacent bf16 values as floats, and back (round to nearest even).
-__device__ __forceinline__ f32x4 bf4_f32(const uint2& w) {
-  float x0, x1, x2, x3;
-  unpack_bf16x2(w.x, x0, x1);
-  unpack_bf16x2(w.y, x2, x3);
-  return f32x4{x0, x1, x2, x3};
-}
-
-__device__ __forceinline__ void st_bf4(uint16_t* p, const f32x4& x) {
-  *reinterpret_cast<uint2*>(p) = uint2{cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3])};
-}
-
 __device__ __forceinline__ bf16x8_t as_bf8(const uint4& w) { return __builtin_bit_cast(bf16x8_t, w); }
 
 // c + x . y for two packed bf16 pairs, in fp32.
@@ -712,15 +805,16 @@ __device__ __forceinline__ float dot2_bf16(uint32_t x, uint32_t y, float c) {
                                          false);
 }
 
-// 4 consecutive values of a gradient row, as fp32 or bf16.
-__device__ __forceinline__ void st_grad(float* p, const f32x4& x) { *reinterpret_cast<f32x4*>(p) = x; }
-__device__ __forceinline__ void st_grad(uint16_t* p, const f32x4& x) { st_bf4(p, x); }
+// 4 consecutive values of a gradient row from element `at` of the buffer, as fp32 or bf16.
+template <typename GradT>
+__device__ __forceinline__ void st_grad(__amdgpu_buffer_rsrc_t rows, int at, const f32x4& x) {
+  if constexpr (std::is_same<GradT, float>::value)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, x), rows, at * 4, 0, 0);
+  else
+    buffer_store_b64(rows, uint32_t(at) * 2u, cvt_pk_bf16(x[0], x[1]), cvt_pk_bf16(x[2], x[3]));
+}
 
-// LDS rows of the gradient kernel: 272 B for [*][128] (the packed 8-byte
-// writes of 16 tokens then hit distinct banks; 288 B, which favours the
-// 16-byte reads instead, is 1% slower), 160 B for [*][64].
-constexpr int GLK = D + 8;
-constexpr int GLC = C + 16;
+constexpr int GLC = C + 16;          // [*][64] bf16 rows of the gradient kernel (160 B)
 
 // What the gate gradients of a training step add (GradT = uint16_t): da, db
 // (bf16, [T, HV]) in place of dg, dbeta, and per (chunk slot, v-head) the
@@ -739,12 +833,12 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     int slots, const int2* __restrict__ chunks, const uint16_t* __restrict__ tmrec, const uint16_t* __restrict__ dh,
     GradT* __restrict__ dq, GradT* __restrict__ dk, GradT* __restrict__ dv, GateOut go) {
   constexpr bool kStep = std::is_same<GradT, uint16_t>::value;
-  __shared__ __align__(16) uint16_t sK[C * GLK];
-  __shared__ __align__(16) uint16_t sQ[C * GLK];
-  __shared__ __align__(16) uint16_t sdO[C * GLK];
-  __shared__ __align__(16) uint16_t sVn[C * GLK];   // X; then Vn
-  __shared__ __align__(16) uint16_t sdX[C * GLK];   // dVn; then dX
-  __shared__ __align__(16) uint16_t sS[D * GLK];    // S; then dSn
+  __shared__ __align__(16) uint16_t sK[C * LDK];
+  __shared__ __align__(16) uint16_t sQ[C * LDK];
+  __shared__ __align__(16) uint16_t sdO[C * LDK];
+  __shared__ __align__(16) uint16_t sVn[C * LDK];   // X; then Vn
+  __shared__ __align__(16) uint16_t sdX[C * LDK];   // dVn; then dX
+  __shared__ __align__(16) uint16_t sS[D * LDK];    // S; then dSn
   __shared__ __align__(16) uint16_t sP[C * GLC];    // P; then dPm
   __shared__ __align__(16) uint16_t sB[C * GLC];    // Tm; then dAb + dAb^T
   __shared__ __align__(16) float gbuf[2][GB_SZ + (kStep ? 3 * C : 0)];
@@ -783,18 +877,15 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     const int slot = x.unit / HQ, hq = x.unit - slot * HQ, hv = hq * G + x.m;
     const size_t rec = size_t(slot) * HV + hv;
     if (x.m == 0) {
-      rows_fetch(r.k, k + size_t(hq) * D, size_t(HQ) * D, x.t0, x.len, tid);
-      rows_fetch(r.q, q + size_t(hq) * D, size_t(HQ) * D, x.t0, x.len, tid);
+      rows_fetch<kGradThreads>(r.k, head_rows(k, HQ, hq, x.t0, x.len), HQ, tid);
+      rows_fetch<kGradThreads>(r.q, head_rows(q, HQ, hq, x.t0, x.len), HQ, tid);
     }
-    rows_fetch(r.o, d_out + size_t(hv) * D, size_t(HV) * D, x.t0, x.len, tid);
+    rows_fetch<kGradThreads>(r.o, head_rows(d_out, HV, hv, x.t0, x.len), HV, tid);
     r.tm = reinterpret_cast<const uint4*>(tmrec + rec * C * C)[tid];
+    const auto vb = head_rows(v, HV, hv, x.t0, x.len);
 #pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
-      const int t = 16 * tb + (lane & 15);
-      r.v[tb] = t < x.len ? *reinterpret_cast<const uint2*>(v + (size_t(x.t0 + t) * HV + hv) * D +
-                                                            16 * wave + 4 * (lane >> 4))
-                          : uint2{0, 0};
-    }
+    for (int tb = 0; tb < 4; ++tb)
+      r.v[tb] = buffer_load_b64(vb, uint32_t((16 * tb + (lane & 15)) * HV * D + 16 * wave + 4 * (lane >> 4)) * 2u);
   };
   // this wave's 16 rows of a state record (S or dSn) as MFMA operands
   auto fetch_state = [&](const At& x, const uint16_t* rec0, uint4 (&r)[4], int lane) {
@@ -812,7 +903,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
   auto gates = [&](const GateIn& gi, int len, int lane, float* gb) {
     chunk_gates_calc(gi, len, lane, gb);
     if constexpr (kStep) {
-      const GateFactors f = gate_factors(gi.a + gi.dt, gi.b, expf(gi.alog));
+      const GateFactors f = gate_factors(bf16_bits_to_f32(gi.a) + gi.dt, bf16_bits_to_f32(gi.b), expf(gi.alog));
       gb[GB_DA + lane] = f.da;
       gb[GB_DB + lane] = f.db;
       gb[GB_G + lane] = f.g;
@@ -850,15 +941,11 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     float* gb = gbuf[it & 1];
 
     // P0: rows to LDS
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int x = tid + i * kGradThreads, r = x >> 4, cc = (x & 15) * 8;
-      if (m == 0) {
-        *reinterpret_cast<uint4*>(sK + r * GLK + cc) = cur.k[i];
-        *reinterpret_cast<uint4*>(sQ + r * GLK + cc) = cur.q[i];
-      }
-      *reinterpret_cast<uint4*>(sdO + r * GLK + cc) = cur.o[i];
+    if (m == 0) {
+      rows_store<kGradThreads>(sK, cur.k, tid);
+      rows_store<kGradThreads>(sQ, cur.q, tid);
     }
+    rows_store<kGradThreads>(sdO, cur.o, tid);
     *reinterpret_cast<uint4*>(sB + (tid >> 3) * GLC + 8 * (tid & 7)) = cur.tm;
     lds_barrier();
 
@@ -870,7 +957,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       kd[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const bf16x8_t ko = op_mr(sK, GLK, 16 * tb, 32 * s, lane);
+        const bf16x8_t ko = op_mr(sK, LDK, 16 * tb, 32 * s, lane);
         ks[tb] = mfma16_bf(as_bf8(cur.s[s]), ko, ks[tb]);
         kd[tb] = mfma16_bf(as_bf8(cur.ds[s]), ko, kd[tb]);
       }
@@ -878,7 +965,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     float dot = 0.f;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * GLK + 32 * s + 8 * g) = cur.s[s];
+      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * LDK + 32 * s + 8 * g) = cur.s[s];
       const uint32_t ss[4] = {cur.s[s].x, cur.s[s].y, cur.s[s].z, cur.s[s].w};
       const uint32_t dd[4] = {cur.ds[s].x, cur.ds[s].y, cur.ds[s].z, cur.ds[s].w};
 #pragma unroll
@@ -901,9 +988,9 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
         for (int j = 0; j < n; ++j) {
           int ti, tj;
           tile_of(j, ti, tj);
-          const bf16x8_t ka = op_mr(sK, GLK, 16 * tj, 32 * s, lane);
-          qk[j] = mfma16_bf(ka, op_mr(sQ, GLK, 16 * ti, 32 * s, lane), qk[j]);
-          kk[j] = mfma16_bf(ka, op_mr(sK, GLK, 16 * ti, 32 * s, lane), kk[j]);
+          const bf16x8_t ka = op_mr(sK, LDK, 16 * tj, 32 * s, lane);
+          qk[j] = mfma16_bf(ka, op_mr(sQ, LDK, 16 * ti, 32 * s, lane), qk[j]);
+          kk[j] = mfma16_bf(ka, op_mr(sK, LDK, 16 * ti, 32 * s, lane), kk[j]);
         }
 #pragma unroll
       for (int j = 0; j < n; ++j) {
@@ -929,18 +1016,20 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     ++nx.m;
     if (nx.m == G) nx = seek(at.unit + int(gridDim.x));
     const bool more = nx.unit < units;
+    const At ld = more ? nx : at;       // what is loaded next (the last step loads its own inputs again)
     GateIn gin{};
-    if (wave == 1 && more) gin = gate_in(nx, lane);
+    if (wave == 1) gin = gate_in(ld, lane);
     lds_barrier();
 
     // P2: everything split along v (this wave's 16 rows of the transposed tiles)
     fresh_lane();
     {
       const int v0 = 16 * wave + 4 * g;     // first of this lane's 4 columns v
+      const auto dv_rows = head_rows(dv, HV, hv, t0, len);
       f32x4 xr[4], vn[4], dx[4];
       bf16x8_t xo[2], yo[2];
 #pragma unroll
-      for (int s = 0; s < 2; ++s) yo[s] = op_rm(sdO, GLK, 16 * wave, 32 * s, lane);
+      for (int s = 0; s < 2; ++s) yo[s] = op_rm(sdO, LDK, 16 * wave, 32 * s, lane);
 #pragma unroll
       for (int tb = 0; tb < 4; ++tb) {
         const int t = 16 * tb + c;
@@ -954,20 +1043,20 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           x[i] = be * xr[tb][i];
           kd[tb][i] *= dc;
         }
-        st_bf4(sVn + t * GLK + v0, x);
+        st_bf4(sVn + t * LDK + v0, x);
         // dVn = Dc K dSn^T + P^T dO
         dx[tb] = kd[tb];
 #pragma unroll
         for (int s = tb / 2; s < 2; ++s)
           dx[tb] = mfma16_bf(yo[s], op_rm(sP, GLC, 16 * tb, 32 * s, lane), dx[tb]);
-        st_bf4(sdX + t * GLK + v0, dx[tb]);
+        st_bf4(sdX + t * LDK + v0, dx[tb]);
       }
       // Vn = Tm X and dX = Tm^T dVn (Tm lower: rows 0-31 of Tm need only their
       // own 32 columns, rows 32-63 of Tm^T likewise)
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        xo[s] = op_rm(sVn, GLK, 16 * wave, 32 * s, lane);
-        yo[s] = op_rm(sdX, GLK, 16 * wave, 32 * s, lane);
+        xo[s] = op_rm(sVn, LDK, 16 * wave, 32 * s, lane);
+        yo[s] = op_rm(sdX, LDK, 16 * wave, 32 * s, lane);
       }
 #pragma unroll
       for (int tb = 0; tb < 4; ++tb) {
@@ -983,8 +1072,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       for (int tb = 0; tb < 4; ++tb) {
         const int t = 16 * tb + c;
         const float be = gb[GB_BETA + t];
-        st_bf4(sVn + t * GLK + v0, vn[tb]);
-        st_bf4(sdX + t * GLK + v0, dx[tb]);
+        st_bf4(sVn + t * LDK + v0, vn[tb]);
+        st_bf4(sdX + t * LDK + v0, dx[tb]);
         f32x4 dvv;
         float sg = 0.f, sb = 0.f, sv = 0.f;
 #pragma unroll
@@ -994,7 +1083,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           sg = fmaf(dvv[i], ks[tb][i], sg);
           sv = fmaf(vn[tb][i], kd[tb][i], sv);
         }
-        if (t < len) st_grad(dv + (size_t(t0 + t) * HV + hv) * D + v0, dvv);
+        st_grad<GradT>(dv_rows, t * HV * D + v0, dvv);
         vks += sv;
         sg = group4_sum(-sg - sv);
         sb = group4_sum(sb);
@@ -1011,7 +1100,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     fresh_lane();
     // the next step's inputs are loaded over P3 and P4
     Regs nxt;
-    if (more) fetch(nx, nxt, tid, lane);
+    fetch(ld, nxt, tid, lane);
     // P3: dP and dA tiles (rows s = 16 tj + 4 g + i, column t = 16 ti + c)
     auto da_tiles = [&](auto count) {
       constexpr int n = decltype(count)::value;
@@ -1024,9 +1113,9 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
         for (int j = 0; j < n; ++j) {
           int ti, tj;
           tile_of(j, ti, tj);
-          const bf16x8_t va = op_mr(sVn, GLK, 16 * tj, 32 * s, lane);
-          dp[j] = mfma16_bf(va, op_mr(sdO, GLK, 16 * ti, 32 * s, lane), dp[j]);
-          da[j] = mfma16_bf(va, op_mr(sdX, GLK, 16 * ti, 32 * s, lane), da[j]);
+          const bf16x8_t va = op_mr(sVn, LDK, 16 * tj, 32 * s, lane);
+          dp[j] = mfma16_bf(va, op_mr(sdO, LDK, 16 * ti, 32 * s, lane), dp[j]);
+          da[j] = mfma16_bf(va, op_mr(sdX, LDK, 16 * ti, 32 * s, lane), da[j]);
         }
 #pragma unroll
       for (int j = 0; j < n; ++j) {
@@ -1076,9 +1165,9 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     };
     if (wave >= 6) da_tiles(IC<2>());
     else da_tiles(IC<1>());
-    if (wave == 1 && more) gates(gin, nx.len, lane, gbuf[(it + 1) & 1]);
+    if (wave == 1) gates(gin, ld.len, lane, gbuf[(it + 1) & 1]);
     lds_barrier();
-    if (more) fetch_state(nx, h, nxt.s, lane);
+    fetch_state(ld, h, nxt.s, lane);
     // P4: dQ = scale E dO S + dPm K;  dK = Dc Vn dSn - beta E dX S + dPm^T Q + (dAb + dAb^T) K
     fresh_lane();
     const int tr0 = 32 * (wave & 1), k0 = 32 * (wave >> 1);
@@ -1092,9 +1181,9 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       bf16x8_t so[2], oo[2], xo[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        so[u] = op_rm(sS, GLK, k0 + 16 * u, 32 * s, lane);
-        oo[u] = op_mr(sdO, GLK, tr0 + 16 * u, 32 * s, lane);
-        xo[u] = op_mr(sdX, GLK, tr0 + 16 * u, 32 * s, lane);
+        so[u] = op_rm(sS, LDK, k0 + 16 * u, 32 * s, lane);
+        oo[u] = op_mr(sdO, LDK, tr0 + 16 * u, 32 * s, lane);
+        xo[u] = op_mr(sdX, LDK, tr0 + 16 * u, 32 * s, lane);
       }
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
@@ -1113,7 +1202,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       float sq = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        const f32x4 qv = bf4_f32(*reinterpret_cast<const uint2*>(sQ + t * GLK + k0 + 16 * kb + 4 * g));
+        const f32x4 qv = bf4_f32(*reinterpret_cast<const uint2*>(sQ + t * LDK + k0 + 16 * kb + 4 * g));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           y[kb][tb][i] *= fq;
@@ -1131,7 +1220,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       const bool lo = s == 0 || tr0 != 0, hi = s == 1 || tr0 == 0;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        ko[u] = op_rm(sK, GLK, k0 + 16 * u, 32 * s, lane);
+        ko[u] = op_rm(sK, LDK, k0 + 16 * u, 32 * s, lane);
         bo[u] = op_mr(sB, GLC, tr0 + 16 * u, 32 * s, lane);
       }
       if (lo) {
@@ -1145,7 +1234,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       if (hi) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          qo[u] = op_rm(sQ, GLK, k0 + 16 * u, 32 * s, lane);
+          qo[u] = op_rm(sQ, LDK, k0 + 16 * u, 32 * s, lane);
           pto[u] = op_rm(sP, GLC, tr0 + 16 * u, 32 * s, lane);
         }
 #pragma unroll
@@ -1161,8 +1250,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     lds_barrier();
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * GLK + 32 * s + 8 * g) = cur.ds[s];
-    if (more) fetch_state(nx, dh, nxt.ds, lane);
+      *reinterpret_cast<uint4*>(sS + (16 * wave + c) * LDK + 32 * s + 8 * g) = cur.ds[s];
+    fetch_state(ld, dh, nxt.ds, lane);
     lds_barrier();
     fresh_lane();
     {
@@ -1176,8 +1265,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
         bf16x8_t so[2], vo[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          so[u] = op_rm(sS, GLK, k0 + 16 * u, 32 * s, lane);
-          vo[u] = op_mr(sVn, GLK, tr0 + 16 * u, 32 * s, lane);
+          so[u] = op_rm(sS, LDK, k0 + 16 * u, 32 * s, lane);
+          vo[u] = op_mr(sVn, LDK, tr0 + 16 * u, 32 * s, lane);
         }
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -1196,19 +1285,18 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
         }
       }
     }
-    if (m == G - 1) {
+    // the last v-head stores the sums (the buffers are empty before it)
+    {
+      const int n = m == G - 1 ? len : 0;
+      const auto dq_rows = head_rows(dq, HQ, hq, t0, n), dk_rows = head_rows(dk, HQ, hq, t0, n);
 #pragma unroll
-      for (int tb = 0; tb < 2; ++tb) {
-        const int t = tr0 + 16 * tb + c;
-        if (t < len) {
-          const size_t row = (size_t(t0 + t) * HQ + hq) * D + k0 + 4 * g;
+      for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            st_grad(dq + row + 16 * kb, dq_acc[kb][tb]);
-            st_grad(dk + row + 16 * kb, dk_acc[kb][tb]);
-          }
+        for (int kb = 0; kb < 2; ++kb) {
+          const int at0 = (tr0 + 16 * tb + c) * HQ * D + k0 + 16 * kb + 4 * g;
+          st_grad<GradT>(dq_rows, at0, dq_acc[kb][tb]);
+          st_grad<GradT>(dk_rows, at0, dk_acc[kb][tb]);
         }
-      }
     }
     if (wave == 0) {
       const int t = lane, blk = lane >> 4;
@@ -1347,12 +1435,14 @@ int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const fl
   const int cus = device_cus();
   const size_t wgs = size_t(cus > 0 ? cus : 256);
   if (N > 0) {
-    // Persistent workgroups, one per CU, when each takes many units (the next
-    // unit's inputs are then fetched during the current one); with few units
-    // per CU, one workgroup per unit, which the dispatcher balances.
-    const unsigned pgrid = unsigned(units >= 8 * wgs ? wgs : units);
-    hipLaunchKernelGGL((gdn_bwd_prep_kernel<CuT>), dim3(pgrid), dim3(kGradThreads), 0, st, q, k, A_log, a,
-                       dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h_chunks, int(slots), w.m, w.r, w.tm, w.chunks);
+    // Two persistent workgroups per CU.  A unit takes the v-heads of a qk-head
+    // together (K, Q and their products once) where that leaves every
+    // workgroup a unit; with fewer, a v-head each.
+    const int heads = slots * size_t(HQ) >= 2 * wgs ? HV / HQ : 1;
+    const unsigned pgrid = unsigned(std::min(slots * size_t(HV / heads), 2 * wgs));
+    hipLaunchKernelGGL((gdn_bwd_prep_kernel<CuT>), dim3(pgrid), dim3(kPrepThreads), 0, st, q, k, A_log, a,
+                       dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h_chunks, int(slots), heads, w.m, w.r,
+                       w.tm, w.chunks);
     // The reverse chain: one workgroup of 8 waves per chain, or, when the
     // chains leave most CUs idle, 4 workgroups of 2 waves (32 state rows) each.
     const unsigned chain_ids = 8u * ((unsigned(N) * unsigned(HV) + 7u) / 8u);
