@@ -46,3 +46,37 @@ def test_step_equals_separate_calls(device, lens, HQ, HV, with_state, dfin, cu32
     size = bwd.gdn_gate_backward(*gates, want["dg"].abs(), want["dbeta"])
     for got, name in ((dA_log, "dA_log"), (ddt_bias, "ddt_bias")):
         assert bool(((got - gate[name]).abs() <= 2 * T * 2.0 ** -24 * size[name].abs()).all()), name
+
+
+# 1 to 9 chunks: each remainder of the ring of four buffers, and past it
+@pytest.mark.parametrize("group,name", [(1, "8 workgroups per chain"), (8, "4 workgroups per chain")])
+def test_chain_kernels_agree(device, group, name):
+    """A sequence's gradients do not depend on the batch it is in: alone (8
+    chains) or with seven others (64) its chains run on the kernels for few
+    chains, in a batch of nine (72) on the general one, with the same
+    operations in the same order."""
+    inp, pre, bwd = (pkg_module(n) for n in ("inputs", "prefill", "backward"))
+    lens = [64 * n - (n % 3) for n in range(1, 10)]
+    print(f"backward chains, {name}", flush=True)
+    x = inp.prefill_inputs(lens, 4, 8, seed=41, with_state=True)
+    g = {k: (v.to(device) if torch.is_tensor(v) else v) for k, v in x.items()}
+    gen = torch.Generator(device=device).manual_seed(19)
+    d_out = torch.randn(sum(lens), 8, 128, generator=gen, device=device).to(torch.bfloat16)
+    d_fin = torch.randn(len(lens), 8, 128, 128, generator=gen, device=device) * 0.1
+
+    def grads(first, last):
+        lo, hi = int(x["cu_seqlens"][first]), int(x["cu_seqlens"][last])
+        q, k, v, a, b = (g[n][lo:hi] for n in ("q", "k", "v", "a", "b"))
+        cu = (x["cu_seqlens"][first:last + 1] - lo).to(device)
+        gates = (g["A_log"], a, g["dt_bias"], b)
+        # the fused kernel's states for every batch: the split path's differ in rare last places
+        _, _, h = pre.gdn_prefill_h(q, k, v, g["state"][first:last], *gates, cu, g["scale"], path="fused")
+        return bwd.gdn_prefill_backward(q, k, v, *gates, cu, g["scale"], h, d_out[lo:hi], d_fin[first:last]), lo, hi
+
+    whole, _, _ = grads(0, len(lens))
+    for first in range(0, len(lens) - group + 1, group):
+        part, lo, hi = grads(first, first + group)
+        torch.cuda.synchronize()
+        for n in ("dq", "dk", "dv", "dg", "dbeta"):
+            assert torch.equal(part[n], whole[n][lo:hi]), (n, first)
+        assert torch.equal(part["dh0"], whole["dh0"][first:first + group]), first

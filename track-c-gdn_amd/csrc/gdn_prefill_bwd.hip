@@ -616,49 +616,90 @@ __global__ __launch_bounds__(kPrepThreads, 2) void gdn_bwd_prep_kernel(
 // ---------------------------------------------------------------------------
 // 2. The state-gradient chain per (sequence, v-head), last chunk first:
 //    dS = dSn M + R, dSn (bf16 [v][k]) over the chunk's R record;  finally dh0 = dS.
-// The 16 rows of dSn that a wave writes are the bytes of the R block that only
-// it reads, and it has them in registers by then.
-// NW waves per workgroup, 128 / (16 NW) workgroups per chain.  A wave keeps
-// dS^T[k][v] for its 16 state rows v as 8 accumulator tiles (k blocks); the
-// B operand of step s is the pair of tiles kt = 2 s, 2 s + 1.
-template <typename CuT, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
+// A wave keeps dS^T[k][v] for 16 state rows v as 8 accumulator tiles (k
+// blocks); the B operand of step s is the pair of tiles kt = 2 s, 2 s + 1.
+// The rows of dS evolve independently (dS = dSn M + R row by row).  The 16
+// rows of dSn that a wave writes are the bytes of the R block that only it
+// reads, and it has them in registers by then.
+struct ChainLane {
+  int vb;              // 16-row block of the state this wave holds
+  int g, c, lane;
+  size_t state;        // element offset of this lane's state row in a [N, HV, 128, 128] tensor
+  uint32_t line;       // byte offset of this lane's pieces in whole-line stores of a 16-row tile
+};
+
+__device__ __forceinline__ ChainLane chain_lane(int vb, int n, int HV, int hv, int lane) {
+  const int g = lane >> 4, c = lane & 15;
+  return ChainLane{vb, g, c, lane, ((size_t(n) * HV + hv) * D + 16 * vb + c) * D, state_lines_lane(g, c)};
+}
+
+__device__ __forceinline__ void chain_load(f32x4 (&acc)[8], const float* d_ht, const ChainLane& w) {
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt)
+    acc[kt] = d_ht ? *reinterpret_cast<const f32x4*>(d_ht + w.state + 16 * kt + 4 * w.g)
+                   : f32x4{0.f, 0.f, 0.f, 0.f};
+}
+
+__device__ __forceinline__ void chain_fetch_r(uint4 (&r)[4], const char* rec, const ChainLane& w) {
+#pragma unroll
+  for (int kp = 0; kp < 4; ++kp)
+    r[kp] = *reinterpret_cast<const uint4*>(rec + ((w.vb * 4 + kp) * 64 + w.lane) * 16);
+}
+
+// dSn as the B operand of the product.
+__device__ __forceinline__ void chain_pack(bf16x8_t (&bop)[4], const f32x4 (&acc)[8]) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) bop[s] = pack2_bf(acc[2 * s], acc[2 * s + 1]);
+}
+
+// dSn to its record as whole 128-byte lines.
+__device__ __forceinline__ void chain_put(const bf16x8_t (&bop)[4], char* rec, const ChainLane& w) {
+#pragma unroll
+  for (int pp = 0; pp < 2; ++pp) {
+    u32x4_t d1, d2;
+    state_lines(w.c, bop[2 * pp], bop[2 * pp + 1], d1, d2);
+    char* p = rec + w.vb * 4096 + 128 * pp + w.line;
+    *reinterpret_cast<u32x4_t*>(p) = d1;
+    *reinterpret_cast<u32x4_t*>(p + 8 * D * 2) = d2;
+  }
+}
+
+__device__ __forceinline__ f32x4 chain_r_tile(const uint4 (&r)[4], int kt) {
+  return bf4_f32((kt & 1) ? uint2{r[kt / 2].z, r[kt / 2].w} : uint2{r[kt / 2].x, r[kt / 2].y});
+}
+
+__device__ __forceinline__ void chain_store(float* dh0, const f32x4 (&acc)[8], const ChainLane& w) {
+  if (dh0) {
+#pragma unroll
+    for (int kt = 0; kt < 8; ++kt)
+      *reinterpret_cast<f32x4*>(dh0 + w.state + 16 * kt + 4 * w.g) = acc[kt];
+  }
+}
+
+// One workgroup of 8 waves per chain: M through LDS, copied (and R loaded into
+// registers) two chunks ahead by the waves themselves.  Bound by HBM while
+// the chains fill the chip: 96 KB per chunk and chain (32 768 tokens qk16/v32:
+// 328 us; 376 us with dSn stored in 8-byte pieces of half lines).
+template <typename CuT>
+__global__ __launch_bounds__(512, 1) void gdn_bwd_chain_kernel(
     const CuT* __restrict__ cu, int N, int T, int HV, int h_chunks, const char* __restrict__ mrec,
     char* rrec, const float* __restrict__ d_ht, float* __restrict__ dh0) {
-  constexpr int S = 8 / NW;                    // slices (of 16 NW state rows) per chain
-  constexpr int kThreads = 64 * NW;
+  constexpr int kThreads = 512;
   __shared__ __align__(16) uint16_t sM[3][D * D];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // Workgroup -> (chain = (sequence, v-head), slice).  The rows of dS evolve
-  // independently (dS = dSn M + R row by row), so a chain splits over S
-  // workgroups that never exchange data; its slices get ids 8 apart, which
-  // puts them on one XCD, so M is read from HBM once per chain.
-  const int xcd = blockIdx.x & 7, id_row = blockIdx.x >> 3;
-  const int chain = 8 * (id_row / S) + xcd;
-  if (chain >= N * HV) return;
-  const int slice = id_row - (id_row / S) * S;
-  const int n = chain / HV, hv = chain - n * HV;
+  const int n = int(blockIdx.x) / HV, hv = int(blockIdx.x) - n * HV;
   int bos, slen;
   seq_bounds(cu, n, T, bos, slen);
   const int nc = (slen + C - 1) / C;
   const int coff = chunk_offset(cu, n, T, lane);
-  const int g = lane >> 4, c = lane & 15;
-  const int vb = slice * NW + wave;            // 16-row block of the state this wave holds
-  const int v = 16 * vb + c;                   // state row (v) of this lane's accumulator column
-
+  const ChainLane w = chain_lane(wave, n, HV, hv, lane);
   f32x4 acc[8];
-#pragma unroll
-  for (int kt = 0; kt < 8; ++kt) {
-    const int k0 = 16 * kt + 4 * g;
-    acc[kt] = d_ht ? *reinterpret_cast<const f32x4*>(d_ht + ((size_t(n) * HV + hv) * D + v) * D + k0)
-                   : f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  chain_load(acc, d_ht, w);
   int last = nc - 1;
   if (coff + last >= h_chunks) last = -1;     // records at or past h_chunks (clamped to the workspace's slots) were not formed
-  // M is copied HBM -> LDS and R loaded into registers two chunks ahead: three
-  // LDS buffers for M and three register sets for R, rotated by unrolling the
-  // chunk loop by three.
+  // three LDS buffers for M and three register sets for R, rotated by
+  // unrolling the chunk loop by three
   constexpr int kMCopies = int(kMBytes / 16) / kThreads;
   auto rec_of = [&](int ch) { return size_t(coff + ch) * HV + hv; };
   auto copy_m = [&](int ch, int buf) {
@@ -667,12 +708,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     for (int x = 0; x < kMCopies; ++x)
       lds_dma16_saddr(ms, uint32_t((x * kThreads + tid) * 16), &sM[buf][(x * kThreads + wave * 64) * 8]);
   };
-  auto fetch_r = [&](int ch, uint4 (&r)[4]) {
-    const char* rs = rrec + rec_of(ch) * kRBytes;
-#pragma unroll
-    for (int kp = 0; kp < 4; ++kp)
-      r[kp] = *reinterpret_cast<const uint4*>(rs + ((vb * 4 + kp) * 64 + lane) * 16);
-  };
+  auto fetch_r = [&](int ch, uint4 (&r)[4]) { chain_fetch_r(r, rrec + rec_of(ch) * kRBytes, w); };
   // one chunk: dSn out, dS = dSn M + R (cur = R of chunk ch), and the copies
   // for chunk ch - 2 (R into nxt2, M into LDS buffer (it + 2) % 3)
   auto step = [&](int ch, int it, uint4 (&cur)[4], uint4 (&nxt2)[4]) {
@@ -681,29 +717,21 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
       copy_m(ch - 2, (it + 2) % 3);
       fetch_r(ch - 2, nxt2);
     }
-    uint16_t* hd = reinterpret_cast<uint16_t*>(rrec + rec_of(ch) * kRBytes);
-#pragma unroll
-    for (int kt = 0; kt < 8; ++kt) {
-      uint2 w;
-      w.x = pack_bf16x2(acc[kt][0], acc[kt][1]);
-      w.y = pack_bf16x2(acc[kt][2], acc[kt][3]);
-      *reinterpret_cast<uint2*>(hd + v * D + 16 * kt + 4 * g) = w;
-    }
     bf16x8_t bop[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) bop[s] = pack2_bf(acc[2 * s], acc[2 * s + 1]);
+    chain_pack(bop, acc);
+    chain_put(bop, rrec + rec_of(ch) * kRBytes, w);
 #pragma unroll
     for (int kt = 0; kt < 8; ++kt) {
-      acc[kt] = bf4_f32((kt & 1) ? uint2{cur[kt / 2].z, cur[kt / 2].w} : uint2{cur[kt / 2].x, cur[kt / 2].y});
+      acc[kt] = chain_r_tile(cur, kt);
 #pragma unroll
       for (int s = 0; s < 4; ++s)
         acc[kt] = mfma16_bf(ld16_bf(&sM[buf][((kt * 4 + s) * 64 + lane) * 8]), bop[s], acc[kt]);
     }
     // Vector memory operations complete in issue order: with at most this
-    // chunk's copies (M and R two chunks ahead) and its 8 dSn stores still
+    // chunk's copies (M and R two chunks ahead) and its 4 dSn stores still
     // outstanding, everything the next chunk reads has landed.
-    if (ch > 1) wait_vm<kMCopies + 4 + 8>();
-    else wait_vm<8>();
+    if (ch > 1) wait_vm<kMCopies + 4 + 4>();
+    else wait_vm<4>();
     lds_barrier();
   };
   uint4 r0[4], r1[4], r2[4];
@@ -722,11 +750,137 @@ __global__ __launch_bounds__(64 * NW, 1) void gdn_bwd_chain_kernel(
     if (ch >= 1) step(ch - 1, it + 1, r1, r0);
     if (ch >= 2) step(ch - 2, it + 2, r2, r1);
   }
-  if (dh0) {
+  chain_store(dh0, acc, w);
+}
+
+// When the chains leave most CUs idle: 8 / NR workgroups per chain, NR waves
+// of 16 state rows in each, and the latency of one chunk's step is what
+// counts.  kCopyWaves more waves copy M into a ring of four LDS buffers, up to four
+// chunks ahead, and store dSn, which the row waves leave in LDS.  A row wave
+// has the chunk's M operands in registers before the chunk begins: behind the
+// products of each half of the k blocks it reads the next chunk's operands,
+// so its step is 32 products with the reads under them.  4096 tokens qk4/v8
+// (64 chunks, 8 chains), us per launch: 86 with the kernel above cut to two
+// waves (16 copies, 32 reads, 8 stores and 32 products in a row); 51 with copy
+// waves and the row waves' own whole-line stores (56 with 8-byte pieces).
+constexpr int kRing = 4, kCopyWaves = 2;
+
+template <typename CuT, int NR>
+__global__ __launch_bounds__(64 * (NR + kCopyWaves), 1) void gdn_bwd_chain_few_kernel(
+    const CuT* __restrict__ cu, int N, int T, int HV, int h_chunks, const char* __restrict__ mrec,
+    char* rrec, const float* __restrict__ d_ht, float* __restrict__ dh0) {
+  constexpr int kSlices = 8 / NR;
+  __shared__ __align__(16) uint16_t sM[kRing][D * D];
+  __shared__ __align__(16) uint16_t sOut[2][16 * NR * LDK];   // dSn of the even and odd steps
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Workgroup -> (chain = (sequence, v-head), slice of 16 NR state rows): a
+  // chain's slices get ids 8 apart, which puts them on one XCD, so M is read
+  // from HBM once per chain.
+  const int xcd = blockIdx.x & 7, id_row = blockIdx.x >> 3;
+  const int chain = 8 * (id_row / kSlices) + xcd, slice = id_row % kSlices;
+  if (chain >= N * HV) return;
+  const int n = chain / HV, hv = chain - n * HV;
+  int bos, slen;
+  seq_bounds(cu, n, T, bos, slen);
+  const int nc = (slen + C - 1) / C;
+  const int coff = chunk_offset(cu, n, T, lane);
+  int last = nc - 1;
+  if (coff + last >= h_chunks) last = -1;     // as above
+  auto rec_of = [&](int ch) { return size_t(coff + ch) * HV + hv; };
+  if (wave >= NR) {
+    constexpr int kCopies = int(kMBytes / 1024) / kCopyWaves, kStores = 4 * NR / kCopyWaves;
+    const int part = wave - NR;               // of M and of dSn
+    auto copy_m = [&](int ch, int buf) {
+      const char* ms = mrec + rec_of(ch) * kMBytes + part * (kCopies * 1024);
 #pragma unroll
-    for (int kt = 0; kt < 8; ++kt)
-      *reinterpret_cast<f32x4*>(dh0 + ((size_t(n) * HV + hv) * D + v) * D + 16 * kt + 4 * g) = acc[kt];
+      for (int x = 0; x < kCopies; ++x)
+        lds_dma16_saddr(ms, uint32_t(x * 1024 + lane * 16), &sM[buf][(part * kCopies + x) * 512]);
+    };
+    auto store_out = [&](int ch, int parity) {
+      char* out = rrec + rec_of(ch) * kRBytes + slice * NR * 4096;
+#pragma unroll
+      for (int x = 0; x < kStores; ++x) {
+        const int at = (part * kStores + x) * 64 + lane;        // 16-byte piece of the rows
+        *reinterpret_cast<uint4*>(out + at * 16) =
+            *reinterpret_cast<const uint4*>(&sOut[parity][(at >> 4) * LDK + (at & 15) * 8]);
+      }
+    };
+#pragma unroll
+    for (int x = 0; x < kRing; ++x)
+      if (last - x >= 0) copy_m(last - x, x);
+    wait_vm<0>();
+    lds_barrier();                            // A: the first four chunks have landed
+    lds_barrier();                            // B: chunk `last` is in registers
+    for (int ch = last, it = 0; ch >= 0; --ch, ++it) {
+      // chunk ch - 4 over chunk ch, and the step before's dSn to its record;
+      // chunk ch - 2 has landed when the step ends (operations complete in
+      // issue order: behind its copies come at most those of two more chunks
+      // and the stores of two steps)
+      if (ch >= 4) copy_m(ch - 4, it & 3);
+      if (it > 0) store_out(ch + 1, (it - 1) & 1);
+      if (ch >= 4) wait_vm<2 * (kCopies + kStores)>();
+      else wait_vm<0>();
+      lds_barrier();
+    }
+    if (last >= 0) store_out(0, last & 1);
+    return;
   }
+  const ChainLane w = chain_lane(NR * slice + wave, n, HV, hv, lane);
+  f32x4 acc[8];
+  chain_load(acc, d_ht, w);
+  bf16x8_t m[8][4];
+  uint4 r[kRing][4];
+#pragma unroll
+  for (int x = 0; x < kRing - 1; ++x)
+    if (last - x >= 0) chain_fetch_r(r[x], rrec + rec_of(last - x) * kRBytes, w);
+  lds_barrier();                              // A
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) m[kt][s] = ld16_bf(&sM[0][((kt * 4 + s) * 64 + lane) * 8]);
+  lds_barrier();                              // B
+  // chunk ch (step it): R in r[x], x = it % 4, the next chunk's M in buffer
+  // (it + 1) % 4; past the first chunk the records read are chunk 0's, whose
+  // values are not used
+  auto step = [&](int ch, auto slot) {
+    constexpr int x = decltype(slot)::value, nb = (x + 1) % kRing;
+    chain_fetch_r(r[(x + 3) % kRing], rrec + rec_of(max(ch - 3, 0)) * kRBytes, w);
+    bf16x8_t bop[4];
+    chain_pack(bop, acc);
+    // one address for the buffer's reads (the compiler would form one per read)
+    uint32_t at = uint32_t(nb * D * D + lane * 8);
+    asm volatile("" : "+v"(at));
+    const uint16_t* next = &sM[0][0] + at;
+    uint16_t* out = &sOut[x & 1][(16 * wave + w.c) * LDK + 4 * w.g];
+#pragma unroll
+    for (int kt = 0; kt < 8; kt += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[kt + u] = chain_r_tile(r[x], kt + u);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[kt + u] = mfma16_bf(m[kt + u][s], bop[s], acc[kt + u]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) m[kt + u][s] = ld16_bf(next + ((kt + u) * 4 + s) * 512);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint4 p = __builtin_bit_cast(uint4, bop[kt / 2 + u]);
+        *reinterpret_cast<uint2*>(out + 16 * (kt + 2 * u)) = uint2{p.x, p.y};
+        *reinterpret_cast<uint2*>(out + 16 * (kt + 2 * u + 1)) = uint2{p.z, p.w};
+      }
+    }
+    lds_barrier();
+  };
+  for (int ch = last; ch >= 0; ch -= 4) {
+    step(ch, IC<0>());
+    if (ch >= 1) step(ch - 1, IC<1>());
+    if (ch >= 2) step(ch - 2, IC<2>());
+    if (ch >= 3) step(ch - 3, IC<3>());
+  }
+  chain_store(dh0, acc, w);
 }
 
 // Gradients of one token's gating
@@ -1443,15 +1597,20 @@ int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const fl
     hipLaunchKernelGGL((gdn_bwd_prep_kernel<CuT>), dim3(pgrid), dim3(kPrepThreads), 0, st, q, k, A_log, a,
                        dt_bias, b, cu, N, T, HQ, HV, scale, d_out, h_chunks, int(slots), heads, w.m, w.r,
                        w.tm, w.chunks);
-    // The reverse chain: one workgroup of 8 waves per chain, or, when the
-    // chains leave most CUs idle, 4 workgroups of 2 waves (32 state rows) each.
-    const unsigned chain_ids = 8u * ((unsigned(N) * unsigned(HV) + 7u) / 8u);
-    if (cus > 0 && 4LL * N * HV <= cus)
-      hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 2>), dim3(4u * chain_ids), dim3(128), 0, st, cu, N, T,
-                         HV, h_chunks, w.m, w.r, d_ht, dh0);
-    else
-      hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT, 8>), dim3(chain_ids), dim3(512), 0, st, cu, N, T, HV,
+    // The reverse chain: one workgroup per chain, or eight or four where they
+    // all run at once (a chain's time is then its chunks' latency, which more
+    // workgroups of fewer rows cut; with more chains than that HBM bounds the
+    // launch).
+    const unsigned chains = unsigned(N) * unsigned(HV), chain_ids = 8u * ((chains + 7u) / 8u);
+    if (cus > 0 && 8LL * N * HV <= cus)
+      hipLaunchKernelGGL((gdn_bwd_chain_few_kernel<CuT, 1>), dim3(8u * chain_ids), dim3(64 * (1 + kCopyWaves)), 0, st, cu, N, T, HV,
                          h_chunks, w.m, w.r, d_ht, dh0);
+    else if (cus > 0 && 4LL * N * HV <= cus)
+      hipLaunchKernelGGL((gdn_bwd_chain_few_kernel<CuT, 2>), dim3(4u * chain_ids), dim3(64 * (2 + kCopyWaves)), 0, st, cu, N, T, HV,
+                         h_chunks, w.m, w.r, d_ht, dh0);
+    else
+      hipLaunchKernelGGL((gdn_bwd_chain_kernel<CuT>), dim3(chains), dim3(512), 0, st, cu, N, T, HV, h_chunks,
+                         w.m, w.r, d_ht, dh0);
     if (T > 0) {
       // one workgroup per CU walks the (chunk, qk-head) units
       const unsigned ggrid = unsigned(std::min(slots * size_t(HQ), wgs));

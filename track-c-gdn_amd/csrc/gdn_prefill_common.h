@@ -223,8 +223,8 @@ __device__ __forceinline__ void buffer_store_b64(__amdgpu_buffer_rsrc_t r, uint3
 __device__ __forceinline__ uint32_t state_lines_lane(int g, int c) {
   return uint32_t((c & 7) * 128 + ((g & 1) ? 4 * (g + 3) : 4 * g)) * 2u + ((c & 8) ? 64u : 0u);
 }
-__device__ __forceinline__ void store_state_lines(char* tile, uint32_t lane_off, int c, bf16x8_t s0,
-                                                  bf16x8_t s1) {
+// (state_lines forms the two stores' data; the second goes 8 rows below the first.)
+__device__ __forceinline__ void state_lines(int c, bf16x8_t s0, bf16x8_t s1, u32x4_t& d1, u32x4_t& d2) {
   const u32x4_t w0 = __builtin_bit_cast(u32x4_t, s0);
   const u32x4_t w1 = __builtin_bit_cast(u32x4_t, s1);
   const auto a0 = __builtin_amdgcn_permlane16_swap(w0[0], w0[2], false, false);
@@ -234,7 +234,6 @@ __device__ __forceinline__ void store_state_lines(char* tile, uint32_t lane_off,
   const uint32_t x[4] = {a0[0], a1[0], a0[1], a1[1]};
   const uint32_t y[4] = {b0[0], b1[0], b0[1], b1[1]};
   const bool low = (c & 8) == 0;
-  u32x4_t d1, d2;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const uint32_t rx = __builtin_amdgcn_update_dpp(0u, x[e], 0x128, 0xf, 0xf, false);   // row_ror:8
@@ -242,6 +241,11 @@ __device__ __forceinline__ void store_state_lines(char* tile, uint32_t lane_off,
     d1[e] = low ? x[e] : ry;
     d2[e] = low ? rx : y[e];
   }
+}
+__device__ __forceinline__ void store_state_lines(char* tile, uint32_t lane_off, int c, bf16x8_t s0,
+                                                  bf16x8_t s1) {
+  u32x4_t d1, d2;
+  state_lines(c, s0, s1, d1, d2);
   store_b128_saddr(tile, lane_off, d1);
   store_b128_saddr(tile, lane_off + 8u * 128u * 2u, d2);
 }
