@@ -170,10 +170,8 @@ class _GatedDeltaRule(torch.autograd.Function):
         if d_o is None:
             d_o = torch.zeros(v.shape, dtype=torch.bfloat16, device=v.device)
         # the forward takes bf16 q, k, v, a, b and fp32 A_log, dt_bias, state only
-        with torch.no_grad():
-            grads = _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, ctx.scale, h, d_o,
-                                   d_final, ctx.has_state)
-        return grads + (None, None)
+        return _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, ctx.scale, h, d_o, d_final,
+                              ctx.has_state) + (None, None)
 
 
 def chunk_gated_delta_rule(q, k, v, A_log, a, dt_bias, b, cu_seqlens, initial_state=None,

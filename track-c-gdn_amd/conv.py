@@ -38,7 +38,6 @@ def _weights(weight, bias, C):
     return weight, bias
 
 
-@torch.no_grad()
 def qkv_conv1d(mixed_qkv, weight, bias, cu_seqlens, conv_state=None, *, num_q_heads: int,
                num_v_heads: int, activation: Optional[str] = "silu", state_len: Optional[int] = None,
                return_state: bool = True):
@@ -81,7 +80,6 @@ def qkv_conv1d(mixed_qkv, weight, bias, cu_seqlens, conv_state=None, *, num_q_he
     return q, k, v, final
 
 
-@torch.no_grad()
 def qkv_conv1d_update(mixed_qkv, conv_state, weight, bias, *, num_q_heads: int, num_v_heads: int,
                       slot_ids=None, activation: Optional[str] = "silu"):
     """One decode token per sequence: ``mixed_qkv [B, C]`` (or ``[B, 1, C]``)

@@ -16,6 +16,13 @@ Host-side mirror of the reference decode entry point
 
 All compute runs in the HIP kernel of libgdn_hip.so on torch's current
 stream; there is no CPU path.
+
+At small batches the call itself is what counts (one sequence, qk4 / v8: the
+kernel takes 3.7 us, the launch 3.6 us of host time and the two result
+allocations 2.5 us), so the checks read each tensor's shape and type once and
+convert nothing that already has its type.  No entry point needs a no-grad
+guard (1 us per call): no torch operation reads the inputs unless a type or a
+layout has to change, and the results are new tensors without a graph.
 """
 
 from __future__ import annotations
@@ -39,15 +46,20 @@ def _resolve_scale(scale, head_dim: int) -> float:
     return float(scale)
 
 
+_BF16 = torch.bfloat16
+_F32 = torch.float32
+
+
 def _check_common(q, k, v, A_log, a, dt_bias, b):
     assert q.is_cuda and k.is_cuda and v.is_cuda, "decode inputs must be GPU tensors"
-    assert q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16
-    assert a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16
-    B, T1, nq, d = q.shape
+    assert q.dtype is _BF16 and k.dtype is _BF16 and v.dtype is _BF16
+    assert a.dtype is _BF16 and b.dtype is _BF16
+    qs, vs = q.shape, v.shape
+    B, T1, nq, d = qs
     assert T1 == 1 and d == D
-    assert k.shape == q.shape
-    assert v.dim() == 4 and v.shape[0] == B and v.shape[1] == 1 and v.shape[3] == D
-    nv = v.shape[2]
+    assert k.shape == qs
+    assert len(vs) == 4 and vs[0] == B and vs[1] == 1 and vs[3] == D
+    nv = vs[2]
     assert nv % nq == 0, "v-heads must be a multiple of qk-heads"
     assert A_log.numel() == nv and dt_bias.numel() == nv
     assert a.numel() == B * nv and b.numel() == B * nv
@@ -56,7 +68,11 @@ def _check_common(q, k, v, A_log, a, dt_bias, b):
 
 def _gates(A_log, dt_bias):
     # DEC:131-133 (A_log.float(), dt_bias.float())
-    return A_log.float().contiguous(), dt_bias.float().contiguous()
+    if A_log.dtype is not _F32:
+        A_log = A_log.float()
+    if dt_bias.dtype is not _F32:
+        dt_bias = dt_bias.float()
+    return A_log.contiguous(), dt_bias.contiguous()
 
 
 def _launch(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state, B, nq, nv,
@@ -68,13 +84,13 @@ def _launch(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state, B, n
     a = a.contiguous()
     b = b.contiguous()
     rc = _capi.lib().gdn_decode_ex_fwd(
-        _capi.ptr(q), _capi.ptr(k), _capi.ptr(v), _capi.ptr(state), _capi.ptr(new_state),
-        _capi.ptr(A_log), _capi.ptr(a), _capi.ptr(dt_bias), _capi.ptr(b), _capi.ptr(output),
-        B, nq, nv, float(scale), flags, _capi.stream_handle(q.device))
-    _capi.check(rc, "gdn_decode_ex_fwd")
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), 0 if state is None else state.data_ptr(),
+        new_state.data_ptr(), A_log.data_ptr(), a.data_ptr(), dt_bias.data_ptr(), b.data_ptr(),
+        output.data_ptr(), B, nq, nv, scale, flags, _capi.stream_handle(q.device))
+    if rc:
+        _capi.check(rc, "gdn_decode_ex_fwd")
 
 
-@torch.no_grad()
 def gdn_decode(q, k, v, state, A_log, a, dt_bias, b, scale=None, *, output=None,
                new_state=None, qk_l2norm: bool = False):
     """One decode step for any ``HV % HQ == 0`` head layout.
@@ -92,27 +108,27 @@ def gdn_decode(q, k, v, state, A_log, a, dt_bias, b, scale=None, *, output=None,
 
 def _decode_impl(q, k, v, state, A_log, a, dt_bias, b, scale=None, *, output=None,
                  new_state=None, qk_l2norm: bool = False):
-    """:func:`gdn_decode` without its no-grad wrapper (the callers hold one)."""
     B, nq, nv = _check_common(q, k, v, A_log, a, dt_bias, b)
     scale = _resolve_scale(scale, q.shape[-1])
     if state is not None:
-        assert state.is_cuda and state.dtype == torch.float32
+        assert state.is_cuda and state.dtype is _F32
         assert state.shape == (B, nv, D, D)
         if not state.is_contiguous():   # DEC:95-96
             state = state.contiguous()
     if output is None:
-        output = torch.empty(B, 1, nv, D, dtype=q.dtype, device=q.device)
+        output = torch.empty((B, 1, nv, D), dtype=_BF16, device=q.device)
+    else:
+        assert output.dtype is _BF16 and output.is_contiguous() and output.numel() == B * nv * D
     if new_state is None:
-        new_state = torch.empty(B, nv, D, D, dtype=torch.float32, device=q.device)
-    assert output.dtype == torch.bfloat16 and output.is_contiguous() and output.numel() == B * nv * D
-    assert new_state.dtype == torch.float32 and new_state.is_contiguous()
-    assert new_state.shape == (B, nv, D, D)
+        new_state = torch.empty((B, nv, D, D), dtype=_F32, device=q.device)
+    else:
+        assert new_state.dtype is _F32 and new_state.is_contiguous()
+        assert new_state.shape == (B, nv, D, D)
     _launch(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state, B, nq, nv,
             _capi.GDN_QK_L2NORM if qk_l2norm else 0)
     return output, new_state
 
 
-@torch.no_grad()
 def run(q, k, v, state, A_log, a, dt_bias, b, scale):
     """Reference-compatible decode entry (DEC:100-146), qk4 / v8 / d128.
 
@@ -127,6 +143,9 @@ def run(q, k, v, state, A_log, a, dt_bias, b, scale):
     assert v.shape[1:] == (1, HV, D)
     assert q.shape[0] == v.shape[0]
     out_dtype = q.dtype
+    if (out_dtype is _BF16 and k.dtype is _BF16 and v.dtype is _BF16 and a.dtype is _BF16
+            and b.dtype is _BF16):
+        return _decode_impl(q, k, v, state, A_log, a, dt_bias, b, scale)
     assert out_dtype.is_floating_point
     q, k, v, a, b = (t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)
                      for t in (q, k, v, a, b))
@@ -134,7 +153,6 @@ def run(q, k, v, state, A_log, a, dt_bias, b, scale):
     return (o if out_dtype == torch.bfloat16 else o.to(out_dtype)), s
 
 
-@torch.no_grad()
 def run_dps(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state):
     """Destination-passing decode: writes ``output`` and ``new_state``, returns None."""
     assert q.shape[1:] == (1, HQ, D)
@@ -144,7 +162,6 @@ def run_dps(q, k, v, state, A_log, a, dt_bias, b, scale, output, new_state):
     _decode_impl(q, k, v, state, A_log, a, dt_bias, b, scale, output=output, new_state=new_state)
 
 
-@torch.no_grad()
 def gdn_decode_multi(q, k, v, state, A_log, a, dt_bias, b, scale=None, *, output=None,
                      new_state=None, qk_l2norm: bool = False):
     """T decode steps per sequence, applied in token order, in one launch.
@@ -190,7 +207,6 @@ def gdn_decode_multi(q, k, v, state, A_log, a, dt_bias, b, scale=None, *, output
     return output, new_state
 
 
-@torch.no_grad()
 def decode_pool_(q, k, v, state_pool, slot_ids, A_log, a, dt_bias, b, scale=None, *,
                  output=None, check_slots: bool = False):
     """One decode step against ``state_pool[slot_ids[n]]``, updated in place.

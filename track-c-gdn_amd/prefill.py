@@ -222,7 +222,6 @@ def num_chunks(cu_seqlens: torch.Tensor, T: int) -> int:
     return int(n)
 
 
-@torch.no_grad()
 def gdn_prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale=None, *,
                 output=None, final_state=None, workspace=None, validate: bool = True,
                 qk_l2norm: bool = False, h=None, path: str = "auto", slices: int = 8,
@@ -398,7 +397,6 @@ def _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale=None, *, out
     return output, final_state
 
 
-@torch.no_grad()
 def gdn_prefill_h(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale=None, *,
                   output=None, final_state=None, h=None, workspace=None, qk_l2norm: bool = False,
                   path: str = "auto", slices: int = 8):
@@ -427,7 +425,6 @@ def gdn_prefill_h(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale=None, 
     return o, s, h
 
 
-@torch.no_grad()
 def run(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale):
     """Reference-compatible prefill entry (PRE:1762-1802), qk4 / v8 / d128.
 
@@ -437,7 +434,6 @@ def run(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale):
     return _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, cu_host=cu_host)
 
 
-@torch.no_grad()
 def run_dps(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, final_state):
     """Destination-passing prefill: writes ``output`` / ``final_state``, returns None."""
     cu_host = validate_inputs(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens)
