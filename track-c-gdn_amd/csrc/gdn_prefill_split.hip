@@ -810,23 +810,23 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
 
     // State update with the chunk's K^T fragments (transposing reads, a
     // k-block ahead) and Vd (state waves).
-    auto update = [&](const _Float16* kc, float egL, const f16x8 (&vd)[2]) {
-      auto load_kt = [&](int kb, f16x8 (&dst)[2]) {
-        const int kq = p32(16 * kb + 4 * (c & 3));
+    auto load_kt = [&](const _Float16* kc, int kb, f16x8 (&dst)[2]) {
+      const int kq = p32(16 * kb + 4 * (c & 3));
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const int tr0 = 32 * p + 4 * g + (c >> 2);
-          const f16x4_t lo = ld_tr16(&kc[tr0 * KCLD + kq]);
-          const f16x4_t hi = ld_tr16(&kc[(tr0 + 16) * KCLD + kq]);
-          dst[p] = f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        }
-      };
+      for (int p = 0; p < 2; ++p) {
+        const int tr0 = 32 * p + 4 * g + (c >> 2);
+        const f16x4_t lo = ld_tr16(&kc[tr0 * KCLD + kq]);
+        const f16x4_t hi = ld_tr16(&kc[(tr0 + 16) * KCLD + kq]);
+        dst[p] = f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    };
+    auto update = [&](const _Float16* kc, float egL, const f16x8 (&vd)[2]) {
       f16x8 fa[3][2];
-      load_kt(0, fa[0]);
-      load_kt(1, fa[1]);
+      load_kt(kc, 0, fa[0]);
+      load_kt(kc, 1, fa[1]);
 #pragma unroll
       for (int kb = 0; kb < 8; ++kb) {
-        if (kb + 2 < 8) load_kt(kb + 2, fa[(kb + 2) % 3]);
+        if (kb + 2 < 8) load_kt(kc, kb + 2, fa[(kb + 2) % 3]);
 #pragma unroll
         for (int p = 0; p < 2; ++p) asm volatile("" : "+v"(fa[kb % 3][p]));
         Sacc[kb] *= egL;
@@ -860,6 +860,64 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
         }
       }
     };
+    // ---- X = beta (V - e^gam K S^T) in place of K S^T.  V[16 tb + 4 g + i]
+    //      [v0 + c] by one transposing read per tb: lane 4 mm + j reads
+    //      columns vl + 4 j .. +3 of row 16 tb + 4 g + mm.
+    i16x4_t xv[4];
+    f32x4 xe[4], xb[4];
+    auto load_x = [&](int b) {
+      const float* gx = reinterpret_cast<const float*>(gt[b]);
+      const int mm = c >> 2, col = vl + 4 * (c & 3);
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) {
+        const int t = 16 * tb + 4 * g + mm;
+        xv[tb] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) i16x4_t*)&rv[b][t * R + 8 * ((col >> 3) ^ vslot<VS>(t)) + (col & 7)]);
+        xe[tb] = *reinterpret_cast<const f32x4*>(&gx[G_EG + 16 * tb + 4 * g]);
+        xb[tb] = *reinterpret_cast<const f32x4*>(&gx[G_BETA + 16 * tb + 4 * g]);
+      }
+    };
+    auto apply_x = [&]() {
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          KS[tb][i] = xb[tb][i] * (bf16_bits_to_f32(uint16_t(xv[tb][i] & vmask)) - xe[tb][i] * KS[tb][i]);
+    };
+    // One row group (4 waves, the whole register file to each): the same
+    // products with every operand in registers beforehand.  K^T is read while
+    // the Tm products run; K, V and the gates of the next chunk (staged by the
+    // middle barrier) under the state update, so that X of the next chunk is
+    // formed before the chunk's last barrier.  One 4096-token sequence,
+    // qk4/v8, the slice launch: 38.9 -> 36.7 us, with h 74.7 -> 62.8.  (The
+    // output wave is the longer one behind the middle barrier: blocks of S Q^T
+    // moved there cost 2 us each, its stores put off to the next chunk gain
+    // 0.4 us without h and lose 9 us with it.)
+    f16x8 kt[NRG == 1 ? 8 : 1][2], kn[NRG == 1 ? 4 : 1][4];
+    auto update_regs = [&](float egL, const f16x8 (&vd)[2]) {
+#pragma unroll
+      for (int kb = 0; kb < 8; ++kb) Sacc[kb] *= egL;
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int kb = 0; kb < 8; ++kb) Sacc[kb] = mfma16(kt[kb][p], vd[p], Sacc[kb]);
+    };
+    auto load_kn = [&](const _Float16* kcb) {
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) kn[p][tb] = ld16(&kcb[(16 * tb + c) * KCLD + 32 * p + 8 * g]);
+    };
+    auto ks_regs = [&](f32x4 (&ks_out)[4]) {
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb) ks_out[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const f16x8 sb = pack2(Sacc[2 * p], Sacc[2 * p + 1]);
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) ks_out[tb] = mfma16(kn[p][tb], sb, ks_out[tb]);
+      }
+    };
     // One chunk; b3c (0, 1, 2) is the buffer set as a compile-time constant,
     // so every LDS address is a loop-invariant lane offset plus an immediate.
     auto chunk = [&](auto b3c, auto rolec, int jj) __attribute__((always_inline)) {
@@ -873,24 +931,13 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
       load_frags(min(ch + kAhead, last_ch), fr[(b3 + kAhead) % FR]);
       if constexpr (!kOut) {
         // K S^T of this chunk was formed at the end of the chunk before
-        // ---- X = beta (V - e^gam K S^T).  V[16 tb + 4 g + i][v0 + c] by one
-        //      transposing read per tb: lane 4 mm + j reads columns vl + 4 j
-        //      .. +3 of row 16 tb + 4 g + mm.
-        {
-          const int mm = c >> 2, j = c & 3;
-          const int col = vl + 4 * j;
+        if constexpr (NRG > 1) {
+          load_x(b3);
+          apply_x();
+        }
+        if constexpr (NRG == 1) {
 #pragma unroll
-          for (int tb = 0; tb < 4; ++tb) {
-            const int t = 16 * tb + 4 * g + mm;
-            const i16x4_t vv = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) i16x4_t*)&rv[b3][t * R + 8 * ((col >> 3) ^ vslot<VS>(t)) + (col & 7)]) &
-                i16x4_t{short(vmask), short(vmask), short(vmask), short(vmask)};
-            const f32x4 eg = *reinterpret_cast<const f32x4*>(&gd[G_EG + 16 * tb + 4 * g]);
-            const f32x4 bt = *reinterpret_cast<const f32x4*>(&gd[G_BETA + 16 * tb + 4 * g]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              KS[tb][i] = bt[i] * (bf16_bits_to_f32(uint16_t(vv[i])) - eg[i] * KS[tb][i]);
-          }
+          for (int kb = 0; kb < 8; ++kb) load_kt(kc, kb, kt[kb]);
         }
         // ---- Vn = Tm X in 32-row blocks: Vn_top = T_a X_top, Vn_bot = T_b (X_bot - A_ba Vn_top)
         f16x8 vd[2];
@@ -917,11 +964,22 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
           xch[r][1][lane] = vn1;
         }
         lds_barrier();                          // Vn of every row group in LDS
-        update(kc, egL, vd);
+        if constexpr (NRG == 1) {
+          load_kn(Kc[(b3 + 1) % NB]);           // past the last chunk not used
+          load_x((b3 + 1) % NB);
+          update_regs(egL, vd);
+        } else {
+          update(kc, egL, vd);
+        }
         // the new state's bf16 image for the output wave, and K S^T of the next chunk
 #pragma unroll
         for (int p = 0; p < 4; ++p) sSb[r][p][lane] = pack2_bf(Sacc[2 * p], Sacc[2 * p + 1]);
-        if (jj + 1 < n_chunks) ks_of(Kc[(b3 + 1) % NB], KS);
+        if constexpr (NRG == 1) {
+          ks_regs(KS);
+          apply_x();
+        } else if (jj + 1 < n_chunks) {
+          ks_of(Kc[(b3 + 1) % NB], KS);
+        }
       } else {
         // ---- O^T = S Q^T (transposed output tile: lane (g, c) of OT[tb] holds
         //      token 16 tb + c, state rows v0 + 4 g .. +3)
@@ -1016,7 +1074,13 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
         for (int p = 0; p < 4; ++p) sSb[r][p][lane] = pack2_bf(Sacc[2 * p], Sacc[2 * p + 1]);
       }
       lds_barrier();                            // chunk 0 staged, the initial state's image written
-      if constexpr (!kOut) ks_of(Kc[0], KS);
+      if constexpr (!kOut) {
+        ks_of(Kc[0], KS);
+        if constexpr (NRG == 1) {
+          load_x(0);
+          apply_x();
+        }
+      }
       int ch = 0;
       for (; ch + NB <= n_chunks; ch += NB) {
         chunk(IC<0>{}, rolec, ch);
