@@ -284,10 +284,11 @@ def bench_prefill_h(dev, steps, warmup, name="prefill_varlen8_t32768_qk16_v32", 
     return dict(total_ms=total_ms, kernel_ms=kern_ms, chunks=NT, h_bytes=h.numel() * 2)
 
 
-# MFMA products the backward executes per (64-token chunk, v-head): 656 in the
-# transition kernel, 256 in the reverse chain, 1360 in the gradient kernel,
-# each a 16x16x32 product of 16 384 flops (dense tiles as launched).
-BWD_MFMA_PER_CHUNK_HEAD = 656 + 256 + 1360
+# MFMA products the backward executes per (64-token chunk, v-head), dense bf16
+# 16x16x32 tiles: 568 in the preparation kernel with two v-heads per qk-head
+# in a workgroup (608 with one: K K^T and Q K^T again), 256 in the reverse
+# chain, 1104 in the gradient kernel.
+BWD_MFMA_PER_CHUNK_HEAD = 568 + 256 + 1104
 
 
 def bench_backward(dev, steps, warmup, name="prefill_varlen8_t32768_qk16_v32",
@@ -749,7 +750,7 @@ def main():
                              "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                              "frac": round(tfl / MFMA_BF16_PEAK_TFLOPS, 4),
                              "flops_per_launch": r["flops"],
-                             "flops_basis": "executed bf16 MFMA products, 2272 per chunk and v-head",
+                             "flops_basis": f"executed bf16 MFMA products, {BWD_MFMA_PER_CHUNK_HEAD} per chunk and v-head",
                              "time_basis": "all launches of one call"}}
             if key == "prefill_backward":
                 tr = _traffic("gdn_prefill_bwd_t32768_qk16_v32")
