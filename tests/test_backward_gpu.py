@@ -83,6 +83,32 @@ def test_backward_matches_oracle(device, lens, HQ, HV, with_state, dfin, cu32):
         _check(gg[name], gref[name], name)
 
 
+# chunks whose last row is the chunk's 64th or not, and a sequence of several
+@pytest.mark.parametrize("lens", [[64, 37], [200, 1, 128]])
+def test_backward_with_strong_decay(device, lens):
+    """exp(A_log) from 20 to 148: a token's dg is then far smaller than the
+    state terms of its chunk, which cancel in it.  Every head keeps the bars
+    of the other tests, the per-head sums relative to their terms'
+    magnitudes."""
+    print(f"backward strong decay lens={lens}", flush=True)
+    x, d_out, d_fin = _case(lens, 4, 8, 90 + sum(lens), True, True)
+    x["A_log"] = torch.linspace(3.0, 5.0, 8)
+    g = _to(x, device)
+    r = _gpu_backward(g, d_out, d_fin, device)
+    bwd = pkg_module("backward")
+    gg = bwd.gdn_gate_backward(g["A_log"], g["a"], g["dt_bias"], g["b"], r["dg"], r["dbeta"])
+    torch.cuda.synchronize()
+    ref = O.prefill_backward(*[x[n] for n in NAMES], x["scale"], d_out, d_fin)
+    gref = O.gate_backward(x["A_log"], x["a"], x["dt_bias"], x["b"], ref["dg"], ref["dbeta"])
+    size = O.gate_backward(x["A_log"], x["a"], x["dt_bias"], x["b"], ref["dg"].abs(), ref["dbeta"])
+    for hv in range(8):
+        _check(r["dg"][:, hv], ref["dg"][:, hv], f"dg, head {hv}")
+        _check(gg["da"][:, hv], gref["da"][:, hv], f"da, head {hv}")
+        for name in ("dA_log", "ddt_bias"):
+            err = abs(float(gg[name][hv]) - float(gref[name][hv]))
+            assert err <= REL_BAR * abs(float(size[name][hv])), (name, hv, err)
+
+
 def test_gate_backward_exact_inputs(device):
     """gdn_gate_bwd alone, from the oracle's own dg / dbeta (fp32 rounding only)."""
     bwd = pkg_module("backward")

@@ -941,13 +941,13 @@ __device__ __forceinline__ void sum_pair_256(float& x, float& y, float (&red)[2]
 // summation order).
 struct GradParts {
   float ag[8][C];    // dgam rows of the [64][128] products (contributor: wave)
+  float av[8][C];    // Dc rowsum(Vn K dSn^T) (contributor: wave)
   float ab[8][C];    // dbeta rows of the [64][128] products
-  float tg[4][C];    // dgam rows, [64][64] products (contributor: column block)
+  float tg[4][C];    // dgam rows, [64][64] products below the diagonal (contributor: column block)
   float tb[4][C];    // dbeta rows, [64][64] products
   float tc[4][C];    // dgam column sums (to subtract), [64][64] products (contributor: row block)
   float aq[4][C];    // scale E rowsum(Q (dO S)) (contributor: column quarter)
   float dot[2][8];   // <dSn, S> per wave, by parity of the step
-  float vks[8];      // sum of Dc rowsum(Vn K dSn^T) per wave
 };
 
 __device__ __forceinline__ bf16x8_t as_bf8(const uint4& w) { return __builtin_bit_cast(bf16x8_t, w); }
@@ -1221,7 +1221,6 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           if (s >= tb / 2) dx[tb] = mfma16_bf(yo[s], op_rm(sB, GLC, 16 * tb, 32 * s, lane), dx[tb]);
         }
       }
-      float vks = 0.f;
 #pragma unroll
       for (int tb = 0; tb < 4; ++tb) {
         const int t = 16 * tb + c;
@@ -1238,16 +1237,15 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           sv = fmaf(vn[tb][i], kd[tb][i], sv);
         }
         st_grad<GradT>(dv_rows, t * HV * D + v0, dvv);
-        vks += sv;
-        sg = group4_sum(-sg - sv);
+        sg = group4_sum(-sg);
+        sv = group4_sum(sv);
         sb = group4_sum(sb);
         if (g == 0) {
           pt.ag[wave][t] = sg;
+          pt.av[wave][t] = sv;
           pt.ab[wave][t] = sb;
         }
       }
-      vks = wave_inclusive_scan(vks);
-      if (lane == 63) pt.vks[wave] = vks;
     }
     lds_barrier();
 
@@ -1285,7 +1283,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           dpm[i] = scale * ex[j][i] * dp[j][i];
           const float xa = t > s0 + i ? -ex[j][i] * da[j][i] : 0.f;
           dab[i] = be * xa;
-          cs[i] = fmaf(dpm[i], qk[j][i], dab[i] * kk[j][i]);
+          // (a diagonal term would be added to its row and taken off its column)
+          cs[i] = t > s0 + i ? fmaf(dpm[i], qk[j][i], dab[i] * kk[j][i]) : 0.f;
           rg += cs[i];
           rb = fmaf(xa, kk[j][i], rb);
         }
@@ -1454,13 +1453,13 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
     }
     if (wave == 0) {
       const int t = lane, blk = lane >> 4;
-      float dgam = 0.f, dbt = 0.f, dsum = 0.f, vks = 0.f;
+      float dgam = 0.f, dbt = 0.f, dsum = 0.f, vk = 0.f;
 #pragma unroll
       for (int w = 0; w < 8; ++w) {
         dgam += pt.ag[w][t];
         dbt += pt.ab[w][t];
         dsum += pt.dot[it & 1][w];
-        vks += pt.vks[w];
+        vk += pt.av[w][t];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1471,11 +1470,16 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
         }
         if (j >= blk) dgam -= pt.tc[j][t];
       }
-      if (t == C - 1) dgam += vks + gb[GB_EL] * dsum;
-      // dg_t = sum_{i >= t} dgam_i
-      const float incl = wave_inclusive_scan(dgam);
-      const float total = __shfl(incl, 63);
-      const float dgt = total - incl + dgam;
+      if (t == C - 1) dgam += gb[GB_EL] * dsum;
+      // dg_t = sum_{i >= t} dgam_i.  Of the row terms vk = Dc rowsum(Vn K
+      // dSn^T), taken off each row and added whole to the last one, that
+      // leaves sum_{i < t} vk_i, formed as such: with strong decay dg is far
+      // smaller than the vk of the last rows, and their difference would be
+      // its rounding (A_log 3 to 5: dA_log 2.1e-2 off, 5.9e-3 with both sums in one
+      // order, 2.8e-3 like this).
+      const float suffix = __shfl(wave_inclusive_scan(__shfl(dgam, 63 - t)), 63 - t);
+      const float before = __shfl_up(vk, 1);
+      const float dgt = suffix + wave_inclusive_scan(t == 0 ? 0.f : before);
       const size_t i = size_t(t0 + t) * HV + hv;
       if constexpr (kStep) {
         float sa = 0.f, sd = 0.f;
