@@ -80,3 +80,31 @@ def test_chain_kernels_agree(device, group, name):
         for n in ("dq", "dk", "dv", "dg", "dbeta"):
             assert torch.equal(part[n], whole[n][lo:hi]), (n, first)
         assert torch.equal(part["dh0"], whole["dh0"][first:first + group]), first
+
+
+def _hooked_grads(device, pack, unpack):
+    bwd, inp = pkg_module("backward"), pkg_module("inputs")
+    x = inp.prefill_inputs([70, 9], 2, 4, seed=61, with_state=True)
+    names = ("q", "k", "v", "A_log", "a", "dt_bias", "b")
+    leaves = [x[n].to(device).requires_grad_() for n in names]
+    gen = torch.Generator(device=device).manual_seed(3)
+    d_out = torch.randn(79, 4, 128, generator=gen, device=device).to(torch.bfloat16)
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        o, _ = bwd.chunk_gated_delta_rule(*leaves, x["cu_seqlens"].to(device), x["state"].to(device), x["scale"])
+    return torch.autograd.grad(o, leaves, d_out)
+
+
+def test_saved_tensor_hooks_that_change_types(device):
+    """What a saved-tensor hook hands back in a wider type or another order of
+    memory gives the same gradients bit for bit."""
+    def wider(t):
+        return t.float() if t.dtype == torch.bfloat16 and t.dim() < 4 else t
+
+    def reordered(t):
+        return t.t().contiguous().t() if t.dim() == 2 else t
+
+    print("saved-tensor hooks", flush=True)
+    want = _hooked_grads(device, lambda t: t, lambda t: t)
+    for unpack in (wider, reordered):
+        for got, ref in zip(_hooked_grads(device, lambda t: t, unpack), want):
+            assert got.dtype == ref.dtype and torch.equal(got, ref)

@@ -128,14 +128,28 @@ def _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, scale, h, d_out, d
     """The gradients of one training step in the inputs' own types: the token
     gradients in bf16 (rounded once, where they are formed), ``dA_log``,
     ``ddt_bias`` and the initial state's in fp32."""
-    T, HQ, _ = q.shape
+    T, HQ, d = q.shape
     HV = v.shape[1]
     N = cu_seqlens.numel() - 1
     dev = q.device
-    q, k, v, a, b, A_log, dt_bias, cu, h = (t.contiguous() for t in (q, k, v, a, b, A_log, dt_bias,
-                                                                     cu_seqlens, h))
-    d_out = d_out.to(torch.bfloat16).contiguous()
+    # A saved-tensor hook may hand back other types or devices than the forward saved: inputs of
+    # another float type are converted, the rest is refused before anything reads an address.
+    at = q.get_device()                 # -1 in host memory
+    assert at >= 0 and (at == k.get_device() == v.get_device() == A_log.get_device() == a.get_device()
+                        == dt_bias.get_device() == b.get_device() == cu_seqlens.get_device()
+                        == h.get_device() == d_out.get_device())
+    assert d == HEAD_SIZE and HV % HQ == 0
+    assert k.shape == q.shape and v.shape == d_out.shape == (T, HV, HEAD_SIZE)
+    assert a.shape == b.shape == (T, HV) and A_log.numel() == dt_bias.numel() == HV
+    assert h.dtype is torch.bfloat16 and h.dim() == 4 and h.shape[1:] == (HV, HEAD_SIZE, HEAD_SIZE)
+    assert cu_seqlens.dtype in (torch.int64, torch.int32)
+    q, k, v, a, b, d_out = ((t if t.dtype is torch.bfloat16 else t.to(torch.bfloat16)).contiguous()
+                            for t in (q, k, v, a, b, d_out))
+    A_log, dt_bias = ((t if t.dtype is torch.float32 else t.to(torch.float32)).contiguous()
+                      for t in (A_log, dt_bias))
+    cu, h = cu_seqlens.contiguous(), h.contiguous()
     if d_final_state is not None:
+        assert d_final_state.get_device() == at and d_final_state.shape == (N, HV, HEAD_SIZE, HEAD_SIZE)
         d_final_state = d_final_state.to(torch.float32).contiguous()
     grads = [torch.empty(t.shape, dtype=torch.bfloat16, device=dev) for t in (q, k, v, a, b)]
     dA_log, ddt_bias = (torch.empty(HV, dtype=torch.float32, device=dev) for _ in range(2))
@@ -161,6 +175,7 @@ class _GatedDeltaRule(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, h)
         ctx.scale = _pre._resolve_scale(scale)
         ctx.has_state = initial_state is not None
+        ctx.chunks = h.shape[0]
         ctx.set_materialize_grads(False)       # no zeros for an output without a gradient
         return o, final
 
@@ -169,6 +184,7 @@ class _GatedDeltaRule(torch.autograd.Function):
         q, k, v, A_log, a, dt_bias, b, cu_seqlens, h = ctx.saved_tensors
         if d_o is None:
             d_o = torch.zeros(v.shape, dtype=torch.bfloat16, device=v.device)
+        assert h.shape[0] >= ctx.chunks, "h holds fewer chunks than the batch has"
         # the forward takes bf16 q, k, v, a, b and fp32 A_log, dt_bias, state only
         return _step_backward(q, k, v, A_log, a, dt_bias, b, cu_seqlens, ctx.scale, h, d_o, d_final,
                               ctx.has_state) + (None, None)
