@@ -130,6 +130,9 @@ struct FusedSeams {
 // qk16/v32, us per launch in index order / longest first: 24 sequences of 37
 // to 523 tokens (q/k L2-normalised) 92.8 / 86.7; 32 of 20 000 tokens in all 197.5 / 185.2; 30 of
 // 32 768 (normalised) 349.6 / 319.1; 12 of 12 000 139.3 / 123.3.
+// An instantiation of its own takes it (Order = LaunchOrder; the pack is empty
+// in index order): as an argument of every launch it cost those without an
+// order 0.2 us (one 64-token sequence 11.24 -> 11.44, 33 of them 23.55 -> 23.75).
 constexpr int kMaxLaunchOrder = 64;
 struct LaunchOrder {
   int on;
@@ -140,7 +143,7 @@ struct LaunchOrder {
 // (row offsets dropped), so their copies and waits are the chain's own.
 __device__ __align__(256) uint16_t g_zero_v_row[D];
 
-template <typename CuT, bool kL2, bool kH>
+template <typename CuT, bool kL2, bool kH, typename... Order>
 __global__ __launch_bounds__(kThreads, 1) void gdn_prefill_chain_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const float* __restrict__ h0,
@@ -148,7 +151,8 @@ __global__ __launch_bounds__(kThreads, 1) void gdn_prefill_chain_kernel(
     const float* __restrict__ dt_bias, const uint16_t* __restrict__ b,
     const CuT* __restrict__ cu_seqlens, int N, int T, int HQ, int HV,
     float scale, uint16_t* __restrict__ out, float* __restrict__ ht,
-    uint16_t* __restrict__ hout, int h_chunks, const FusedSeams seams, const LaunchOrder order) {
+    uint16_t* __restrict__ hout, int h_chunks, const FusedSeams seams, const Order... order) {
+  constexpr bool kOrder = sizeof...(Order) > 0;
   __shared__ Smem sm;
   __shared__ SmemRaw raw;
   __shared__ __align__(16) uint16_t rawV[C * D];     // V chunk (bf16, swizzled), DMA target
@@ -175,15 +179,15 @@ __global__ __launch_bounds__(kThreads, 1) void gdn_prefill_chain_kernel(
     // in launch order, rows of 8 units are snaked over the XCDs, which a
     // sequence of fewer than 8 qk-heads fills in part
     const int row = id_row / heads_per_qk;
-    const int unit = 8 * row + (order.on && (row & 1) ? 7 - xcd : xcd);
+    const int unit = 8 * row + (kOrder && (row & 1) ? 7 - xcd : xcd);
     if (unit >= N * HQ) return;
     n = unit / HQ;
     hq = unit - n * HQ;
-    if (order.on) {
+    if constexpr (kOrder) {
       uint64_t w = 0;
 #pragma unroll
       for (int j = 0; j < kMaxLaunchOrder / 8; ++j)
-        if (j == n >> 3) w = order.seq[j];
+        if (j == n >> 3) w = (order.seq[j], ...);
       n = int(w >> (8 * (n & 7))) & 255;
     }
     hv = hq * heads_per_qk + (id_row - (id_row / heads_per_qk) * heads_per_qk);
@@ -1166,31 +1170,31 @@ int check_prefill_args(const void* q, const void* k, const void* v, const void* 
 
 
 // The chain kernel over the chains' grid, plus the seams' workgroups and the
-// seam pass when `seams` holds any (never with h).
-template <bool kL2, bool kH>
+// seam pass when `seams` holds any (never with h or an order).
+template <bool kL2, bool kH, typename... Order>
 int launch_prefill(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* state,
                    const float* A_log, const uint16_t* a, const float* dt_bias, const uint16_t* b,
                    const void* cu_seqlens, int cu_is_int32, int N, int T, int HQ, int HV,
                    float scale, uint16_t* out, float* final_state, uint16_t* h, int h_chunks,
-                   FusedSeams seams, int seam_ox_rows, int seam_max_tail, const LaunchOrder& order,
-                   hipStream_t st) {
+                   FusedSeams seams, int seam_ox_rows, int seam_max_tail, hipStream_t st,
+                   const Order&... order) {
   const unsigned units = unsigned(N) * unsigned(HQ);
   const unsigned G = unsigned(HV / HQ);
   const unsigned base = 8u * G * ((units + 7u) / 8u);
-  if (kH) seams.count = 0;
+  if (kH || sizeof...(Order) > 0) seams.count = 0;
   seams.base_ids = int(base);
   const unsigned seam_units = unsigned(seams.count) * unsigned(HQ);
   const unsigned extra = seams.count > 0 ? 8u * 2u * G * ((seam_units + 7u) / 8u) : 0u;
   const dim3 grid{base + extra, 1u, 1u};
   const dim3 block(kThreads);
   if (cu_is_int32) {
-    hipLaunchKernelGGL((gdn_prefill_chain_kernel<int32_t, kL2, kH>), grid, block, 0, st, q, k, v,
+    hipLaunchKernelGGL((gdn_prefill_chain_kernel<int32_t, kL2, kH, Order...>), grid, block, 0, st, q, k, v,
                        state, A_log, a, dt_bias, b, static_cast<const int32_t*>(cu_seqlens), N, T,
-                       HQ, HV, scale, out, final_state, h, h_chunks, seams, order);
+                       HQ, HV, scale, out, final_state, h, h_chunks, seams, order...);
   } else {
-    hipLaunchKernelGGL((gdn_prefill_chain_kernel<int64_t, kL2, kH>), grid, block, 0, st, q, k, v,
+    hipLaunchKernelGGL((gdn_prefill_chain_kernel<int64_t, kL2, kH, Order...>), grid, block, 0, st, q, k, v,
                        state, A_log, a, dt_bias, b, static_cast<const int64_t*>(cu_seqlens), N, T,
-                       HQ, HV, scale, out, final_state, h, h_chunks, seams, order);
+                       HQ, HV, scale, out, final_state, h, h_chunks, seams, order...);
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return -int(err);
@@ -1208,17 +1212,20 @@ int prefill_dispatch(const uint16_t* q, const uint16_t* k, const uint16_t* v, co
   if (h != nullptr) {
     return l2 ? launch_prefill<true, true>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
                                            cu_is_int32, N, T, HQ, HV, scale, out, final_state, h,
-                                           h_chunks, FusedSeams{}, 0, 0, order, st)
+                                           h_chunks, FusedSeams{}, 0, 0, st)
               : launch_prefill<false, true>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
                                             cu_is_int32, N, T, HQ, HV, scale, out, final_state, h,
-                                            h_chunks, FusedSeams{}, 0, 0, order, st);
+                                            h_chunks, FusedSeams{}, 0, 0, st);
   }
-  return l2 ? launch_prefill<true, false>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
-                                          cu_is_int32, N, T, HQ, HV, scale, out, final_state,
-                                          nullptr, 0, seams, seam_ox_rows, seam_max_tail, order, st)
-            : launch_prefill<false, false>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
-                                           cu_is_int32, N, T, HQ, HV, scale, out, final_state,
-                                           nullptr, 0, seams, seam_ox_rows, seam_max_tail, order, st);
+  auto plain = [&](const auto&... o) {
+    return l2 ? launch_prefill<true, false>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
+                                            cu_is_int32, N, T, HQ, HV, scale, out, final_state,
+                                            nullptr, 0, seams, seam_ox_rows, seam_max_tail, st, o...)
+              : launch_prefill<false, false>(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens,
+                                             cu_is_int32, N, T, HQ, HV, scale, out, final_state,
+                                             nullptr, 0, seams, seam_ox_rows, seam_max_tail, st, o...);
+  };
+  return order.on ? plain(order) : plain();
 }
 
 }  // namespace
