@@ -125,8 +125,9 @@ struct FusedSeams {
 // The order in which a fused launch of more chains than CUs takes the
 // sequences: the longest first, so that the last workgroups to start are the
 // shortest.  Made on the host with the plan, up to kMaxLaunchOrder sequences,
-// where the lengths differ; passed by value, a byte per position (ranked by
-// every workgroup from cu_seqlens instead, it cost each of them 1.3 us).
+// where the modelled finish is earlier by enough (longest_first); passed by
+// value, a byte per position (ranked by every workgroup from cu_seqlens
+// instead, it cost each of them 1.3 us).
 // qk16/v32, us per launch in index order / longest first: 24 sequences of 37
 // to 523 tokens (q/k L2-normalised) 92.8 / 86.7; 32 of 20 000 tokens in all 197.5 / 185.2; 30 of
 // 32 768 (normalised) 349.6 / 319.1; 12 of 12 000 139.3 / 123.3.
@@ -1328,15 +1329,14 @@ constexpr double kStartupCycles = 24000.0;
 constexpr double kSplitStartupCycles = 27700.0;
 constexpr int kFusedSeamMinChunks = 8;    // shortest chain a fused seam cuts
 
-// Finish time of workgroups that each hold one CU for `chunks * period`
-// cycles, started in the given order as CUs free up, `per_seq` workgroups
+// Finish time of workgroups that each hold one CU for their sequence's
+// `times`, started in the given order as CUs free up, `per_seq` workgroups
 // per sequence.  The workgroups of one sequence last equally long, so the
 // CUs are tracked as groups that free at the same time (sorted by time).
-double makespan(const std::vector<int>& chunks, int per_seq, double period, int cus) {
+double makespan(const std::vector<double>& times, int per_seq, int cus) {
   std::vector<std::pair<double, long long>> free_at{{0.0, (long long)cus}};
   double end = 0.0;
-  for (int n : chunks) {
-    const double d = n * period;
+  for (const double d : times) {
     long long need = per_seq;
     while (need > 0 && !free_at.empty()) {
       const double t = free_at.front().first + d;
@@ -1464,7 +1464,10 @@ int choose_path(const CuT* cu, int N, int T, int HQ, int HV, int cus, const Fuse
     int seams = 0;
     const int span = gdn::prefill_split_seam_span(chunks.data(), N, room, &seams);
     // with seams every workgroup is resident: the span is the finish
-    return prep + (seams > 0 ? span * period : makespan(chunks, HV * slices, period, cus));
+    if (seams > 0) return prep + span * period;
+    std::vector<double> times(N);
+    for (int m = 0; m < N; ++m) times[m] = chunks[m] * period;
+    return prep + makespan(times, HV * slices, cus);
   };
   const double split8 = split(8, kSlice8ChunkCycles);
   const double split4 = split(4, kSlice4ChunkCycles);
@@ -1488,8 +1491,19 @@ struct PrefillPlan {
 };
 static_assert(sizeof(PrefillPlan) <= GDN_PREFILL_PLAN_BYTES, "plan size");
 
+// The order is taken where the launch's modelled finish in index order is at
+// least kOrderGain times the one with the longest first, a chain lasting its
+// chunks and kOrderStartupPeriods more.  Below that the order gains nothing
+// and its rounds of equal chains read and write their states all at once: of
+// 220 random batches (5 head layouts, 9 to 64 sequences, 500 to 40 000 tokens)
+// always taking it made 78 slower, by up to 15% (17 sequences of 56 to 166
+// tokens, qk16/v32: 42.0 -> 47.3 us); with this rule 3 are, by at most 2.2%,
+// and the mean gain is 7.1% instead of 6.1%.
+constexpr double kOrderGain = 1.07;
+constexpr double kOrderStartupPeriods = 3.0;
+
 template <typename CuT>
-LaunchOrder longest_first(const CuT* cu, int N, int T) {
+LaunchOrder longest_first(const CuT* cu, int N, int T, int HV, int cus) {
   LaunchOrder o{};
   if (N < 2 || N > kMaxLaunchOrder) return o;
   int chunks[kMaxLaunchOrder], by[kMaxLaunchOrder];
@@ -1500,7 +1514,11 @@ LaunchOrder longest_first(const CuT* cu, int N, int T) {
     by[m] = m;
   }
   std::stable_sort(by, by + N, [&](int x, int y) { return chunks[x] > chunks[y]; });
-  if (chunks[by[0]] == chunks[by[N - 1]]) return o;
+  std::vector<double> d(N);
+  for (int m = 0; m < N; ++m) d[m] = chunks[m] + kOrderStartupPeriods;
+  const double in_index_order = makespan(d, HV, cus);
+  for (int r = 0; r < N; ++r) d[r] = chunks[by[r]] + kOrderStartupPeriods;
+  if (in_index_order < kOrderGain * makespan(d, HV, cus)) return o;
   o.on = 1;
   for (int r = 0; r < N; ++r) o.seq[r >> 3] |= uint64_t(by[r]) << (8 * (r & 7));
   return o;
@@ -1523,7 +1541,7 @@ void make_plan(const CuT* cu, int N, int T, int HQ, int HV, int cus, bool seams,
     p.workspace_bytes = gdn::prefill_split_workspace_bytes(N, T, HQ, HV);
   } else {
     p.workspace_bytes = p.fused.count ? seam_region_bytes(p.fused.count, HV, p.fused.ox_rows) : 0;
-    if (p.fused.count == 0 && cus > 0 && (long long)N * HV > cus) p.order = longest_first(cu, N, T);
+    if (p.fused.count == 0 && cus > 0 && (long long)N * HV > cus) p.order = longest_first(cu, N, T, HV, cus);
   }
 }
 
