@@ -141,6 +141,17 @@ __device__ __forceinline__ float group4_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Three such sums with half the exchanges: x's in lane group 0, y's in group 1
+// (and 3), z's in group 2, each added in group4_sum's order.
+__device__ __forceinline__ float group4_sum3(float x, float y, float z) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(z), false, false);
+  const float xz = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const auto i = __builtin_amdgcn_permlane32_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+  const float yy = __uint_as_float(i[0]) + __uint_as_float(i[1]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(xz), __float_as_uint(yy), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Gate data of one chunk in LDS: gam | beta | e^gam | e^{gam_L - gam} (64 each),
 // then gam_L, e^{gam_L}.  Wave-0 work: lane t takes token t of the chunk.
 constexpr int GB_GAM = 0, GB_BETA = C, GB_E = 2 * C, GB_DC = 3 * C, GB_L = 4 * C, GB_EL = 4 * C + 1;
@@ -940,9 +951,8 @@ __device__ __forceinline__ void sum_pair_256(float& x, float& y, float (&red)[2]
 // Sums over a token's row go through per-contributor partial arrays (fixed
 // summation order).
 struct GradParts {
-  float ag[8][C];    // dgam rows of the [64][128] products (contributor: wave)
-  float av[8][C];    // Dc rowsum(Vn K dSn^T) (contributor: wave)
-  float ab[8][C];    // dbeta rows of the [64][128] products
+  // rows of the [64][128] products (contributor: wave): dgam, dbeta, Dc rowsum(Vn K dSn^T)
+  float row[3][8][C];
   float tg[4][C];    // dgam rows, [64][64] products below the diagonal (contributor: column block)
   float tb[4][C];    // dbeta rows, [64][64] products
   float tc[4][C];    // dgam column sums (to subtract), [64][64] products (contributor: row block)
@@ -1237,14 +1247,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
           sv = fmaf(vn[tb][i], kd[tb][i], sv);
         }
         st_grad<GradT>(dv_rows, t * HV * D + v0, dvv);
-        sg = group4_sum(-sg);
-        sv = group4_sum(sv);
-        sb = group4_sum(sb);
-        if (g == 0) {
-          pt.ag[wave][t] = sg;
-          pt.av[wave][t] = sv;
-          pt.ab[wave][t] = sb;
-        }
+        const float sum = group4_sum3(-sg, sb, sv);
+        if (g < 3) pt.row[g][wave][t] = sum;
       }
     }
     lds_barrier();
@@ -1456,10 +1460,10 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       float dgam = 0.f, dbt = 0.f, dsum = 0.f, vk = 0.f;
 #pragma unroll
       for (int w = 0; w < 8; ++w) {
-        dgam += pt.ag[w][t];
-        dbt += pt.ab[w][t];
+        dgam += pt.row[0][w][t];
+        dbt += pt.row[1][w][t];
         dsum += pt.dot[it & 1][w];
-        vk += pt.av[w][t];
+        vk += pt.row[2][w][t];
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
