@@ -931,13 +931,26 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
       load_frags(min(ch + kAhead, last_ch), fr[(b3 + kAhead) % FR]);
       if constexpr (!kOut) {
         // K S^T of this chunk was formed at the end of the chunk before
-        if constexpr (NRG > 1) {
-          load_x(b3);
-          apply_x();
-        }
         if constexpr (NRG == 1) {
 #pragma unroll
           for (int kb = 0; kb < 8; ++kb) load_kt(kc, kb, kt[kb]);
+        } else {
+          // X a token block at a time (all blocks' operands read beforehand,
+          // as with one row group, made this form 1 to 2% slower)
+          const int mm = c >> 2, j = c & 3;
+          const int col = vl + 4 * j;
+#pragma unroll
+          for (int tb = 0; tb < 4; ++tb) {
+            const int t = 16 * tb + 4 * g + mm;
+            const i16x4_t vv = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) i16x4_t*)&rv[b3][t * R + 8 * ((col >> 3) ^ vslot<VS>(t)) + (col & 7)]) &
+                i16x4_t{short(vmask), short(vmask), short(vmask), short(vmask)};
+            const f32x4 eg = *reinterpret_cast<const f32x4*>(&gd[G_EG + 16 * tb + 4 * g]);
+            const f32x4 bt = *reinterpret_cast<const f32x4*>(&gd[G_BETA + 16 * tb + 4 * g]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              KS[tb][i] = bt[i] * (bf16_bits_to_f32(uint16_t(vv[i])) - eg[i] * KS[tb][i]);
+          }
         }
         // ---- Vn = Tm X in 32-row blocks: Vn_top = T_a X_top, Vn_bot = T_b (X_bot - A_ba Vn_top)
         f16x8 vd[2];
