@@ -879,10 +879,12 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
     };
     auto apply_x = [&]() {
 #pragma unroll
-      for (int tb = 0; tb < 4; ++tb)
+      for (int tb = 0; tb < 4; ++tb) {
+        const i16x4_t vv = xv[tb] & i16x4_t{short(vmask), short(vmask), short(vmask), short(vmask)};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          KS[tb][i] = xb[tb][i] * (bf16_bits_to_f32(uint16_t(xv[tb][i] & vmask)) - xe[tb][i] * KS[tb][i]);
+          KS[tb][i] = xb[tb][i] * (bf16_bits_to_f32(uint16_t(vv[i])) - xe[tb][i] * KS[tb][i]);
+      }
     };
     // One row group (4 waves, the whole register file to each): the same
     // products with every operand in registers beforehand.  K^T is read while
@@ -920,8 +922,15 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
     };
     // One chunk; b3c (0, 1, 2) is the buffer set as a compile-time constant,
     // so every LDS address is a loop-invariant lane offset plus an immediate.
-    auto chunk = [&](auto b3c, auto rolec, int jj) __attribute__((always_inline)) {
+    // tailc: one of the chunks after the loop.  With one row group a last chunk
+    // there ends at its sSb: the next chunk's K S^T and X cost a run of one
+    // chunk 0.25 us (3 sequences of 33 tokens, qk4/v8, replayed from a graph:
+    // 11.38 -> 11.21 us; 8 of 31, qk16/v32, four rounds of slices: 41.6 ->
+    // 40.2).  The loop forms them behind a last chunk too, unused: leaving it
+    // early cost runs of many chunks more.
+    auto chunk = [&](auto b3c, auto rolec, auto tailc, int jj) __attribute__((always_inline)) {
       constexpr int b3 = decltype(b3c)::value;
+      constexpr bool kTail = decltype(tailc)::value != 0;
       constexpr bool kOut = decltype(rolec)::value != 0;
       const int ch = ch0 + jj;                  // the chunk; jj its place in this chain's run
       const int L = chunk_len(ch);
@@ -988,6 +997,10 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
 #pragma unroll
         for (int p = 0; p < 4; ++p) sSb[r][p][lane] = pack2_bf(Sacc[2 * p], Sacc[2 * p + 1]);
         if constexpr (NRG == 1) {
+          if (kTail && jj + 1 == n_chunks) {    // the barrier that ends the chunk
+            lds_barrier();
+            return;
+          }
           ks_regs(KS);
           apply_x();
         } else if (jj + 1 < n_chunks) {
@@ -1096,14 +1109,14 @@ __global__ __launch_bounds__(SliceCfg<NRG>::kThreads, 1) void gdn_prefill_slice_
       }
       int ch = 0;
       for (; ch + NB <= n_chunks; ch += NB) {
-        chunk(IC<0>{}, rolec, ch);
-        chunk(IC<1>{}, rolec, ch + 1);
-        chunk(IC<2>{}, rolec, ch + 2);
-        if constexpr (NB > 3) chunk(IC<(NB > 3 ? 3 : 0)>{}, rolec, ch + 3);
+        chunk(IC<0>{}, rolec, IC<0>{}, ch);
+        chunk(IC<1>{}, rolec, IC<0>{}, ch + 1);
+        chunk(IC<2>{}, rolec, IC<0>{}, ch + 2);
+        if constexpr (NB > 3) chunk(IC<(NB > 3 ? 3 : 0)>{}, rolec, IC<0>{}, ch + 3);
       }
-      if (ch < n_chunks) chunk(IC<0>{}, rolec, ch);
-      if (ch + 1 < n_chunks) chunk(IC<1>{}, rolec, ch + 1);
-      if (NB > 3 && ch + 2 < n_chunks) chunk(IC<2>{}, rolec, ch + 2);
+      if (ch < n_chunks) chunk(IC<0>{}, rolec, IC<1>{}, ch);
+      if (ch + 1 < n_chunks) chunk(IC<1>{}, rolec, IC<1>{}, ch + 1);
+      if (NB > 3 && ch + 2 < n_chunks) chunk(IC<2>{}, rolec, IC<1>{}, ch + 2);
     };
     if (n_chunks > 0) {
       if (out_role) run(IC<1>{});
