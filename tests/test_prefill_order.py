@@ -11,8 +11,6 @@ import torch
 from conftest import pkg_module
 
 CUS = 256
-# the order's place in the opaque plan (layout 2): on, then a byte per position
-ON, SEQ = 216, 224
 
 
 def _plan(lens, HQ, HV, cus=CUS):
@@ -22,20 +20,24 @@ def _plan(lens, HQ, HV, cus=CUS):
     return pre.Plan(cu, sum(lens), HQ, HV, cus=cus)
 
 
-def _order(plan, n):
-    on = struct.unpack_from("i", plan.buf.raw, ON)[0]
-    return list(plan.buf.raw[SEQ:SEQ + n]) if on else None
+def _order(plan, lens):
+    """Where the plan holds these lengths' sequences longest first, a byte each; None: it holds no such run."""
+    chunks = [(n + 63) // 64 for n in lens]
+    order = sorted(range(len(lens)), key=lambda m: -chunks[m])
+    at = plan.buf.raw.find(bytes(order))
+    return None if at < 0 else at
 
 
 def test_order_is_longest_first():
     lens = [64 * ((7 * i) % 10) + i % 3 for i in range(40)]     # chunk counts repeat; some are empty
-    order = _order(_plan(lens, 4, 8), 40)
-    chunks = [(n + 63) // 64 for n in lens]
-    assert order == sorted(range(40), key=lambda m: -chunks[m])
-    assert _order(_plan(lens[:32], 4, 8), 32) is None            # 256 chains on 256 CUs: all start at once
-    assert _order(_plan([100] * 40, 4, 8), 40) is None           # equal lengths
-    assert _order(_plan([60, 70] * 32, 4, 8), 64) is not None
-    assert _order(_plan([60, 70] * 32 + [5], 4, 8), 65) is None  # past what a plan holds
+    def order(lens):
+        return _order(_plan(lens, 4, 8), lens)
+
+    assert order(lens) is not None
+    assert order(lens[:32]) is None                 # 256 chains on 256 CUs: all start at once
+    assert order([100] * 40) is None                # equal lengths
+    assert order([60, 70] * 32) is not None
+    assert order([60, 70] * 32 + [5]) is None       # past what a plan holds
 
 
 # Where longest first saves no round the chains of a round start and end
@@ -47,7 +49,7 @@ def test_order_is_longest_first():
     ([64 * n for n in range(1, 11)], 16, 32, True),      # the longest would start last
     ([64] * 40 + [640], 4, 8, True)])
 def test_order_is_taken_where_it_gains(lens, HQ, HV, ordered):
-    assert (_order(_plan(lens, HQ, HV), len(lens)) is not None) == ordered
+    assert (_order(_plan(lens, HQ, HV), lens) is not None) == ordered
 
 
 def _launch(buf, N, T, HQ=4, HV=8):
@@ -60,7 +62,8 @@ def test_a_plan_that_names_a_sequence_twice_is_refused():
     capi = pkg_module("_capi")
     lens = [64 * (i % 9) + 1 for i in range(40)]
     plan = _plan(lens, 4, 8)
-    for at, value in ((SEQ, plan.buf.raw[SEQ + 1]), (SEQ + 39, 40), (SEQ + 3, 255)):
+    seq = _order(plan, lens)
+    for at, value in ((seq, plan.buf.raw[seq + 1]), (seq + 39, 40), (seq + 3, 255)):
         buf = ctypes.create_string_buffer(plan.buf.raw, capi.GDN_PREFILL_PLAN_BYTES)
         buf[at] = value
         assert _launch(buf, 40, sum(lens)) == capi.GDN_ERR_SHAPE
@@ -91,7 +94,7 @@ def test_results_equal_the_index_order(device, n, HQ, HV, l2):
     x = inp.prefill_inputs(lens, HQ, HV, seed=n, with_state=True)
     g = {k: (v.to(device) if torch.is_tensor(v) else v) for k, v in x.items()}
     args = [g[k] for k in ("q", "k", "v", "state", "A_log", "a", "dt_bias", "b", "cu_seqlens")]
-    assert _order(_plan(lens, HQ, HV, cus=0), n) is not None, "this batch is meant to be ordered"
+    assert _order(_plan(lens, HQ, HV, cus=0), lens) is not None, "this batch is meant to be ordered"
     o, s = pre.gdn_prefill(*args, g["scale"], qk_l2norm=l2)
     o2, s2 = pre.gdn_prefill(*args, g["scale"], qk_l2norm=l2, validate=False)
     torch.cuda.synchronize()
