@@ -284,11 +284,14 @@ def bench_prefill_h(dev, steps, warmup, name="prefill_varlen8_t32768_qk16_v32", 
     return dict(total_ms=total_ms, kernel_ms=kern_ms, chunks=NT, h_bytes=h.numel() * 2)
 
 
-# MFMA products the backward executes per (64-token chunk, v-head), dense bf16
-# 16x16x32 tiles: 568 in the preparation kernel with two v-heads per qk-head
-# in a workgroup (608 with one: K K^T and Q K^T again), 256 in the reverse
-# chain, 1104 in the gradient kernel.
-BWD_MFMA_PER_CHUNK_HEAD = 568 + 256 + 1104
+# bf16 MFMA products (16x16x32 tiles) the backward executes per 64-token chunk
+# and v-head: 528 in the preparation kernel and 80 of K K^T and Q K^T, which
+# the v-heads of a qk-head share where that kernel takes them together (as many
+# units or more as its two workgroups per CU); 256 in the reverse chain; 1104 in
+# the gradient kernel.
+def bwd_mfma_per_chunk_head(T, N, HQ, HV, cus):
+    shared = HV // HQ if (T // 64 + N) * HQ >= 2 * cus else 1
+    return 528 + 80 / shared + 256 + 1104
 
 
 def bench_backward(dev, steps, warmup, name="prefill_varlen8_t32768_qk16_v32",
@@ -322,9 +325,12 @@ def bench_backward(dev, steps, warmup, name="prefill_varlen8_t32768_qk16_v32",
         lib.gdn_prefill_bwd(*call)
 
     total_ms, kern_ms = timed_launches(launch, steps, warmup, warm_ms)
-    flops = h.shape[0] * HV * BWD_MFMA_PER_CHUNK_HEAD * 16384
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    products = bwd_mfma_per_chunk_head(T, N, HQ, HV, cus)
+    flops = int(h.shape[0] * HV * products * 16384)
+    chain = "gdn_bwd_chain_few_kernel" if 4 * N * HV <= cus else "gdn_bwd_chain_kernel"
     return dict(kernel_ms=kern_ms, T=T, N=N, HQ=HQ, HV=HV, chunks=h.shape[0], flops=flops,
-                ws_bytes=need)
+                products=products, chain_kernel=chain, ws_bytes=need)
 
 
 def bench_run_latency(dev, kernel_us, reps=50):
@@ -745,12 +751,12 @@ def main():
                 "workload": name, "tokens": r["T"], "sequences": r["N"], "qk_heads": r["HQ"],
                 "v_heads": r["HV"], "kernel_us": round(kus, 2),
                 "tokens_per_s": round(r["T"] / (r["kernel_ms"] * 1e-3), 1),
-                "kernels": ["gdn_bwd_prep_kernel", "gdn_bwd_chain_kernel", "gdn_bwd_grad_kernel"],
+                "kernels": ["gdn_bwd_prep_kernel", r["chain_kernel"], "gdn_bwd_grad_kernel"],
                 "roofline": {"bound": "mfma", "achieved": round(tfl, 2),
                              "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                              "frac": round(tfl / MFMA_BF16_PEAK_TFLOPS, 4),
                              "flops_per_launch": r["flops"],
-                             "flops_basis": f"executed bf16 MFMA products, {BWD_MFMA_PER_CHUNK_HEAD} per chunk and v-head",
+                             "flops_basis": f"executed bf16 MFMA products, {r['products']:g} per chunk and v-head",
                              "time_basis": "all launches of one call"}}
             if key == "prefill_backward":
                 tr = _traffic("gdn_prefill_bwd_t32768_qk16_v32")
