@@ -14,7 +14,10 @@ of the reference's ``chunk_gated_delta_rule_fwd_h``, PRE:1341-1398).
   inputs ``a, b, A_log, dt_bias`` (``g = -exp(A_log) softplus(a + dt_bias)``,
   ``beta = sigmoid(b)``, PRE:1706-1722).
 * :func:`chunk_gated_delta_rule` -- the prefill as a differentiable torch
-  operator (forward with ``h``, backward through the two calls above).
+  operator.  Its backward is one call of its own (``gdn_prefill_bwd_step``):
+  the kernels of :func:`gdn_prefill_backward`, the token gradients rounded to
+  bf16 where they are formed and taken through the gating there, ``dA_log``
+  and ``ddt_bias`` summed per chunk and then over the chunks in fp32.
 
 All arithmetic runs in the HIP kernels of libgdn_hip.so on torch's current
 stream.  The backward's products take bf16 operands with fp32 accumulation;

@@ -21,8 +21,9 @@
 //     so that dS = dSn M + R.  M is written as ready MFMA A-operand
 //     fragments, R in the accumulator layout of the chain kernel, and Tm for
 //     the gradient kernel.
-//  2. gdn_bwd_chain_kernel, one workgroup per (sequence, v-head), or per
-//     quarter of its state rows when the chains are few: walks the chunks
+//  2. gdn_bwd_chain_kernel, one workgroup per (sequence, v-head), or
+//     gdn_bwd_chain_few_kernel, one per eighth or quarter of its state rows
+//     when the chains are few: walks the chunks
 //     from last to first with dS^T in MFMA accumulators, storing dSn of
 //     every chunk (bf16) and the gradient of the initial state.
 //  3. gdn_bwd_grad_kernel, persistent workgroups over the (chunk, qk-head)
@@ -153,12 +154,13 @@ __device__ __forceinline__ float group4_sum3(float x, float y, float z) {
 }
 
 // Gate data of one chunk in LDS: gam | beta | e^gam | e^{gam_L - gam} (64 each),
-// then gam_L, e^{gam_L}.  Wave-0 work: lane t takes token t of the chunk.
+// then gam_L, e^{gam_L}.  One wave's work (wave 3 of the preparation, wave 1
+// of the gradients): lane t takes token t of the chunk.
 constexpr int GB_GAM = 0, GB_BETA = C, GB_E = 2 * C, GB_DC = 3 * C, GB_L = 4 * C, GB_EL = 4 * C + 1;
 constexpr int GB_SZ = 4 * C + 4;
 constexpr int GB_DA = GB_SZ, GB_DB = GB_SZ + C, GB_G = GB_SZ + 2 * C;   // GateFactors (training step only)
 
-// The gate inputs of token `lane` of the chunk (wave 0): loaded early, used
+// The gate inputs of token `lane` of the chunk: loaded early, used
 // by chunk_gates_calc once the chunk's rows are on their way.
 struct GateIn {
   uint16_t a, b;       // as loaded: converted where they are used, so that nothing waits for them before
@@ -251,10 +253,10 @@ __device__ __forceinline__ void rows_store(uint16_t* dst, const uint4 (&w)[1024 
 // M and like the dSn operand the chain multiplies by M: R enters dS = dSn M +
 // R with the same rounding.
 //
-// Bound by HBM at 32 768 tokens qk16/v32: 0.36 ms for the 2.0 GB it must move
-// (5.6 TB/s).  It replaces a form that took 0.97 ms: one workgroup of 8 waves
-// per CU (160 KB of LDS, scaled copies of K and Q among it) whose other waves
-// waited for one wave's inverse of the whole block.
+// Bound by HBM at 32 768 tokens qk16/v32: 0.35 ms for the 1.75 GB it must move
+// (1.82 GB by the counters, 5.2 TB/s).  It replaces a form that took 0.95 ms:
+// one workgroup of 8 waves per CU (160 KB of LDS, scaled copies of K and Q
+// among it) whose other waves waited for one wave's inverse of the whole block.
 // Workgroups of 4 waves, two per CU (78 KB of LDS each), so that one's serial
 // inverse overlaps the other's products and stores:
 //   P1  the lower 16x16 tiles of A (fp32) and P; wave w inverts A's diagonal
@@ -939,10 +941,11 @@ __device__ __forceinline__ void sum_pair_256(float& x, float& y, float (&red)[2]
 //       Tm^T dVn = dX, Tm X = Vn), their row and column sums
 //   P4  dQ and dK, wave w: tokens 32 (w % 2) .. +31, columns 32 (w / 2) .. +31
 //
-// What bounds it, at 32 768 tokens qk16/v32 (one workgroup per CU, 151 KB of
-// LDS): a step ((chunk, v-head)) takes about 26 000 cycles, of which the VALU
-// is busy 37%, the LDS 41% and the matrix cores 17%; HBM carries 2.5 GB in
-// 0.72 ms.  It replaces a form that took 1.65 ms with the same products split
+// What bounds it, at 32 768 tokens qk16/v32 (one workgroup per CU, 153 KB of
+// LDS): latency within a step ((chunk, v-head)): of its about 24 000 cycles
+// the LDS is busy 46% (42% of that bank conflicts), the VALU 37% and the
+// matrix cores 17%; HBM carries 3.25 GB in 0.74 ms with fp32 gradients, which
+// take 0.70 ms in bf16.  It replaces a form that took 1.65 ms with the same products split
 // by rows over 13 barriers per v-head: there Tm was inverted again by one wave
 // of every workgroup, S and dSn were read from HBM twice, and nothing of the
 // next unit was in flight.  The next step's loads go out over P3 and P4,
@@ -1479,8 +1482,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void gdn_bwd_grad_kernel(
       // dSn^T), taken off each row and added whole to the last one, that
       // leaves sum_{i < t} vk_i, formed as such: with strong decay dg is far
       // smaller than the vk of the last rows, and their difference would be
-      // its rounding (A_log 3 to 5: dA_log 2.1e-2 off, 5.9e-3 with both sums in one
-      // order, 2.8e-3 like this).
+      // its rounding (A_log 3 to 5: dA_log 2.1e-2 off, 5.9e-3 with both sums
+      // in one order, 2.8e-3 like this).
       const float suffix = __shfl(wave_inclusive_scan(__shfl(dgam, 63 - t)), 63 - t);
       const float before = __shfl_up(vk, 1);
       const float dgt = suffix + wave_inclusive_scan(t == 0 ? 0.f : before);
